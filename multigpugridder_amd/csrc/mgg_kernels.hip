@@ -1193,9 +1193,11 @@ __global__ __launch_bounds__(kThreads) void bp_kernel(BPArgs p)
 // The queue spans directions (entries carry a 7-bit direction slot), so the
 // tail of one direction fills up with the next and groups stay full.  Two
 // entries of one group can name the same voxel (different directions), so
-// contributions go to a per-wave LDS accumulator with LDS atomic adds; the
-// four wave accumulators are combined in a fixed order at the end and added
-// to the volume in FP64.
+// contributions go to a per-wave LDS accumulator one direction after the
+// other (plain read-modify-writes: a float LDS atomic holds the LDS for 194
+// cycles per wave, against 8; 7.58 -> 6.92 ms per 2,000 directions at N=128,
+// 2.67 -> 2.29 ms with the density, 777 at N=64); the four wave accumulators
+// are combined in a fixed order at the end and added to the volume in FP64.
 //
 // Table index.  The reference, as contracted, takes
 // k = roundf(fma(clamp(r, -2, 2), 125, 250)) with r = fl(p - v).  For every
@@ -1467,10 +1469,21 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
                             if (DENS) dsum = fmaf(vin[ii], w, dsum);
                         }
                     }
-                    // Two queued entries of one group can name the same voxel
-                    // (different directions): LDS atomic add.
-                    atomicAdd(&sacc[wv][vox], cum);
-                    if (DENS) atomicAdd(&sden[wv][vox], dsum);
+                    // Two queued entries of one group can name the same voxel,
+                    // but only for different directions: the adds go one
+                    // direction after the other, as plain read-modify-writes
+                    // (most groups hold one or two directions).  A wave's LDS
+                    // instructions execute in order.
+                    for (unsigned long long pend = __ballot(true); pend != 0ull;) {
+                        const int first = __builtin_amdgcn_readlane(qq, __builtin_ctzll(pend));
+                        const bool mine = qq == first;
+                        if (mine) {
+                            sacc[wv][vox] += cum;
+                            if (DENS) sden[wv][vox] += dsum;
+                        }
+                        pend &= ~__ballot(mine);
+                        __asm__ volatile("" ::: "memory");
+                    }
                 }
             }
             };
