@@ -182,6 +182,16 @@ int mgg_op_forward_project_checked(const void *cas_volume, int cas_dtype, int v,
 int mgg_op_back_project(float *cas_volume, float *density, int v, const float *axes,
                         int n_axes, const float *cas_images, int m, float mask_radius,
                         const float *ker, int ker_size, float ker_hwidth, void *stream);
+/* mgg_op_back_project with 4 bytes of device scratch, overwritten in stream
+ * order: the call first writes there whether the table's end entries are 0,
+ * table and images are finite and the frames orthonormal; where they are, the
+ * volume is gathered column by column, and the rest as mgg_op_back_project
+ * does (which is also what a NULL scratch asks for).  Same results up to FP32
+ * accumulation order.  No reference counterpart. */
+int mgg_op_back_project_scratch(float *cas_volume, float *density, int v, const float *axes,
+                                int n_axes, const float *cas_images, int m, float mask_radius,
+                                const float *ker, int ker_size, float ker_hwidth, unsigned *scratch,
+                                void *stream);
 /* Exact transpose of mgg_op_forward_project, accumulated into cas_volume
  * (no reference counterpart: the adjoint the autograd backward needs). */
 int mgg_op_back_project_adjoint(float *cas_volume, int v, const float *axes, int n_axes,
@@ -201,6 +211,16 @@ int mgg_op_back_project_adjoint_checked(float *cas_volume, int v, const float *a
                                         const float *cas_images, int m, float mask_radius,
                                         const float *ker, int ker_size, float ker_hwidth,
                                         const unsigned *check, void *stream);
+/* mgg_op_back_project_adjoint_checked with 4 bytes of device scratch,
+ * overwritten in stream order, as mgg_op_back_project_scratch has: where the
+ * table's ends are 0, table and images finite (check says so; NULL: the call
+ * looks) and the frames orthonormal, each voxel gathers its pixels, without
+ * atomics.  Same results up to FP32 accumulation order.  No reference
+ * counterpart. */
+int mgg_op_back_project_adjoint_scratch(float *cas_volume, int v, const float *axes, int n_axes,
+                                        const float *cas_images, int m, float mask_radius,
+                                        const float *ker, int ker_size, float ker_hwidth,
+                                        const unsigned *check, unsigned *scratch, void *stream);
 /* Gridders/gpuGridder.cpp:432-518: n CAS images (m x m) -> images (nn x nn).
  * Uses a batched rocFFT C2R; cas_images is clobbered (used as scratch). */
 int mgg_op_cas_images_to_images(float *cas_images, float *images, int n, int m, int nn,

@@ -94,7 +94,9 @@ _SIGS = {
     "mgg_op_forward_project_checked": [_vp, _ci, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp, _vp],
     "mgg_op_check_volume": [_vp, _ci, _ci, _vp, _ci, _vp, _vp],
     "mgg_op_back_project": [_vp, _vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp],
+    "mgg_op_back_project_scratch": [_vp, _vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp, _vp],
     "mgg_op_back_project_adjoint": [_vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp],
+    "mgg_op_back_project_adjoint_scratch": [_vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp, _vp, _vp],
     "mgg_op_back_project_adjoint_checked": [_vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp, _vp],
     "mgg_op_check_images": [_vp, _ci, _ci, _vp, _ci, _vp, _vp],
     "mgg_op_cas_images_to_images": [_vp, _vp, _ci, _ci, _ci, _vp],

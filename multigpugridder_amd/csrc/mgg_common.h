@@ -125,9 +125,15 @@ void axes_from_normal(const double n[3], double phi_r, float out[9]);
 
 // ---- device chains
 void check_launch(hipError_t e, const char *what);
-const int *brick_order(const ProjGeom &g, int &len);
+const int *brick_order(const ProjGeom &g, int depth, int &len);
+// check: device scratch for launch_check_back's flag, overwritten by the call
+// (stream-ordered); without it every frame takes the voxel-by-voxel kernel.
 hipError_t back_project_launch(float *vol, float *dens, const ProjGeom &g, const float *axes, int n,
-                               const float *casImgs, hipStream_t s);
+                               const float *casImgs, hipStream_t s, unsigned *check = nullptr);
+// finite: launch_check_volume's flag over the images and the table, or null;
+// check: as above.
+hipError_t back_project_adjoint_launch(float *vol, const ProjGeom &g, const float *axes, int n, const float *casImgs,
+                                       hipStream_t s, const unsigned *finite, unsigned *check);
 void chain_cas_to_images(float *casImgs, float2 *herm, float *images, int n, int m, int nn,
                          hipStream_t s);
 // scale / zeroNyq: see launch_herm2d_to_cas (1 / 0 for ImgsToCASImgs itself).

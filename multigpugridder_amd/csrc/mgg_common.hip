@@ -320,21 +320,22 @@ void check_launch(hipError_t e, const char *what)
     if (e != hipSuccess) raise(MGG_ERR_HIP, "%s launch failed: %s", what, hipGetErrorString(e));
 }
 
-// Centre-out brick order of the fast back projection, one device copy per
-// (device, V), built on first use and kept for the process.
+// Centre-out brick orders of the fast and the column back projection, one
+// device copy per (device, V, depth), built on first use and kept for the
+// process.
 std::mutex g_order_mu;
-std::map<std::pair<int, int>, std::unique_ptr<DevBuf>> g_order;
+std::map<std::tuple<int, int, int>, std::unique_ptr<DevBuf>> g_order;
 
-const int *brick_order(const ProjGeom &g, int &len)
+const int *brick_order(const ProjGeom &g, int depth, int &len)
 {
     len = 0;
     if (!bp_uses_fast_path(g)) return nullptr;
-    len = bp_brick_count(g.V, true);
+    len = bp_brick_count(g.V, depth);
     std::lock_guard<std::mutex> lk(g_order_mu);
-    auto &b = g_order[std::make_pair(current_device(), g.V)];
+    auto &b = g_order[std::make_tuple(current_device(), g.V, depth)];
     if (!b) {
         std::vector<int> host(len);
-        bp_brick_order(g.V, host.data());
+        bp_brick_order(g.V, depth, host.data());
         auto nb = std::make_unique<DevBuf>();
         nb->reserve(sizeof(int) * len);
         HIP_TRY(hipMemcpy(nb->ptr, host.data(), sizeof(int) * len, hipMemcpyHostToDevice));
@@ -344,11 +345,40 @@ const int *brick_order(const ProjGeom &g, int &len)
 }
 
 hipError_t back_project_launch(float *vol, float *dens, const ProjGeom &g, const float *axes, int n,
-                               const float *casImgs, hipStream_t s)
+                               const float *casImgs, hipStream_t s, unsigned *check)
 {
     int len = 0;
-    const int *order = brick_order(g, len);
-    return launch_back_project(vol, dens, g, axes, n, casImgs, s, order, len);
+    const int *order = brick_order(g, 8, len);
+    const ColKind kind = ColKind::Back;
+    const bool columns = check != nullptr && dens == nullptr && uses_columns(g, n, kind);
+    if (columns) {
+        int colLen = 0;
+        const int *colOrder = brick_order(g, col_depth(kind), colLen);
+        hipError_t e = launch_check_back(casImgs, g, axes, n, false, check, s);
+        if (e == hipSuccess) e = launch_columns(kind, vol, g, axes, n, casImgs, s, colOrder, colLen, check);
+        if (e != hipSuccess) return e;
+    }
+    return launch_back_project(vol, dens, g, axes, n, casImgs, s, order, len, columns ? check : nullptr);
+}
+
+hipError_t back_project_adjoint_launch(float *vol, const ProjGeom &g, const float *axes, int n, const float *casImgs,
+                                       hipStream_t s, const unsigned *finite, unsigned *check)
+{
+    if (check == nullptr || !uses_columns(g, n, ColKind::Adjoint)) {
+        if (finite == nullptr && check != nullptr) {
+            const hipError_t e = launch_check_volume(casImgs, DT_F32, (size_t)std::max(n, 0) * g.M * g.M, g.ker, g.K,
+                                                     check, s);
+            if (e != hipSuccess) return e;
+            finite = check;
+        }
+        return launch_back_project_adjoint(vol, g, axes, n, casImgs, s, finite);
+    }
+    int len = 0;
+    const int *order = brick_order(g, col_depth(ColKind::Adjoint), len);
+    hipError_t e = launch_check_back(casImgs, g, axes, n, true, check, s, finite);
+    if (e == hipSuccess) e = launch_columns(ColKind::Adjoint, vol, g, axes, n, casImgs, s, order, len, check);
+    if (e != hipSuccess) return e;
+    return launch_back_project_adjoint(vol, g, axes, n, casImgs, s, finite, check);
 }
 
 // CAS images (n x m^2) -> images (n x nn^2); casImgs is reused as the C2R output.

@@ -68,6 +68,7 @@ struct mgg_gridder {
     struct Slot {
         hipStream_t stream = nullptr;
         DevBuf casImgs, herm, imgs, axes;
+        DevBuf check;  // back_project_launch's flag
     };
     std::vector<std::unique_ptr<Slot>> slots;
     // legacy API: library-owned CAS-image output
@@ -288,6 +289,7 @@ struct mgg_gridder {
             Slot &s = *slots[i];
             s.axes.reserve(sizeof(float) * 9 * E);
             s.casImgs.reserve(sizeof(float) * (size_t)E * M * M);
+            s.check.reserve(sizeof(unsigned));
             if (fromImgs) {
                 s.herm.reserve(sizeof(float2) * (size_t)E * M * (M / 2 + 1));
                 s.imgs.reserve(sizeof(float) * (size_t)E * N * N);
@@ -318,7 +320,8 @@ struct mgg_gridder {
                                        sizeof(float) * (size_t)c.count * M * M, hipMemcpyHostToDevice, s.stream));
             }
             check_launch(back_project_launch(parts + V3 * c.slot, withDensity ? partsDens + V3 * c.slot : nullptr, g,
-                                             s.axes.as<float>(), c.count, s.casImgs.as<float>(), s.stream),
+                                             s.axes.as<float>(), c.count, s.casImgs.as<float>(), s.stream,
+                                             s.check.as<unsigned>()),
                          "back_project");
         }
         sync_slots(nS);
@@ -753,9 +756,9 @@ int mgg_op_check_volume(const void *cas_volume, int cas_dtype, int v, const floa
     });
 }
 
-int mgg_op_back_project(float *cas_volume, float *density, int v, const float *axes, int n_axes,
-                        const float *cas_images, int m, float mask_radius, const float *ker, int ker_size,
-                        float ker_hwidth, void *stream)
+int mgg_op_back_project_scratch(float *cas_volume, float *density, int v, const float *axes, int n_axes,
+                                const float *cas_images, int m, float mask_radius, const float *ker, int ker_size,
+                                float ker_hwidth, unsigned *scratch, void *stream)
 {
     return guarded([&] {
         if (n_axes == 0) return;
@@ -763,8 +766,33 @@ int mgg_op_back_project(float *cas_volume, float *density, int v, const float *a
         validate_geom(v, m, ker_size, ker_hwidth);
         if (n_axes < 0) raise(MGG_ERR_INVALID_ARGUMENT, "n_axes < 0");
         ProjGeom g{v, m, mask_radius, ker, ker_size, ker_hwidth};
-        check_launch(back_project_launch(cas_volume, density, g, axes, n_axes, cas_images, as_stream(stream)),
+        check_launch(back_project_launch(cas_volume, density, g, axes, n_axes, cas_images, as_stream(stream), scratch),
                      "back_project");
+    });
+}
+
+int mgg_op_back_project(float *cas_volume, float *density, int v, const float *axes, int n_axes,
+                        const float *cas_images, int m, float mask_radius, const float *ker, int ker_size,
+                        float ker_hwidth, void *stream)
+{
+    return mgg_op_back_project_scratch(cas_volume, density, v, axes, n_axes, cas_images, m, mask_radius, ker, ker_size,
+                                       ker_hwidth, nullptr, stream);
+}
+
+int mgg_op_back_project_adjoint_scratch(float *cas_volume, int v, const float *axes, int n_axes,
+                                        const float *cas_images, int m, float mask_radius, const float *ker,
+                                        int ker_size, float ker_hwidth, const unsigned *check, unsigned *scratch,
+                                        void *stream)
+{
+    return guarded([&] {
+        if (n_axes == 0) return;
+        need(cas_volume, "cas_volume"); need(axes, "axes"); need(cas_images, "cas_images"); need(ker, "ker");
+        validate_geom(v, m, ker_size, ker_hwidth);
+        if (n_axes < 0) raise(MGG_ERR_INVALID_ARGUMENT, "n_axes < 0");
+        ProjGeom g{v, m, mask_radius, ker, ker_size, ker_hwidth};
+        check_launch(back_project_adjoint_launch(cas_volume, g, axes, n_axes, cas_images, as_stream(stream), check,
+                                                 scratch),
+                     "back_project_adjoint");
     });
 }
 
@@ -772,16 +800,8 @@ int mgg_op_back_project_adjoint_checked(float *cas_volume, int v, const float *a
                                         const float *cas_images, int m, float mask_radius, const float *ker,
                                         int ker_size, float ker_hwidth, const unsigned *check, void *stream)
 {
-    return guarded([&] {
-        if (n_axes == 0) return;
-        need(cas_volume, "cas_volume"); need(axes, "axes"); need(cas_images, "cas_images"); need(ker, "ker");
-        validate_geom(v, m, ker_size, ker_hwidth);
-        if (n_axes < 0) raise(MGG_ERR_INVALID_ARGUMENT, "n_axes < 0");
-        ProjGeom g{v, m, mask_radius, ker, ker_size, ker_hwidth};
-        check_launch(launch_back_project_adjoint(cas_volume, g, axes, n_axes, cas_images, as_stream(stream),
-                                                 check),
-                     "back_project_adjoint");
-    });
+    return mgg_op_back_project_adjoint_scratch(cas_volume, v, axes, n_axes, cas_images, m, mask_radius, ker, ker_size,
+                                               ker_hwidth, check, nullptr, stream);
 }
 
 int mgg_op_back_project_adjoint(float *cas_volume, int v, const float *axes, int n_axes,

@@ -41,10 +41,30 @@ hipError_t launch_check_volume(const void *vol, int dtype, size_t n, const float
                                hipStream_t s);
 // Back projection, reference semantics (voxel-owner gather, no atomics).
 // volAcc (V^3) and, if non-null, densAcc (V^3, the plane density = back
-// projection of all-ones CAS images) are accumulated into.
+// projection of all-ones CAS images) are accumulated into.  With check (after
+// launch_columns, fast path only) it does what the columns leave.
 hipError_t launch_back_project(float *volAcc, float *densAcc, const ProjGeom &g,
                                const float *axes, int nAxes, const float *casImgs,
-                               hipStream_t s, const int *brickOrder, int orderLen);
+                               hipStream_t s, const int *brickOrder, int orderLen,
+                               const unsigned *check = nullptr);
+// The same, and the exact transpose (launch_back_project_adjoint), by voxel
+// columns, for the orthonormal frames among the directions when check holds
+// launch_check_back's flag for these images, directions and table (same
+// stream): bit 0, the table's ends are 0 and the table and all image values
+// finite; bit 1, all frames orthonormal.  launch_back_project or
+// launch_back_project_adjoint with the flag must follow.  order is
+// bp_brick_order of depth col_depth(kind).
+enum class ColKind : int { Back = 0, Adjoint = 1 };  // Back: without the density
+// Whether the geometry allows columns and they are the faster way.
+bool uses_columns(const ProjGeom &g, int nAxes, ColKind kind);
+int col_depth(ColKind kind);
+// planes: a frame counts by its first two vectors alone (the transpose).
+// finite: a flag of launch_check_volume over the images and the table, to be
+// used in place of a pass over them.
+hipError_t launch_check_back(const float *casImgs, const ProjGeom &g, const float *axes, int nAxes, bool planes,
+                             unsigned *check, hipStream_t s, const unsigned *finite = nullptr);
+hipError_t launch_columns(ColKind kind, float *volAcc, const ProjGeom &g, const float *axes, int nAxes,
+                          const float *casImgs, hipStream_t s, const int *order, int orderLen, const unsigned *check);
 // Forward projection over several volumes in one launch (FP32 storage, the
 // 501-entry table): each segment is a run of directions on one volume,
 // written to its own CAS images; work items are the segments' 8x8 pixel
@@ -72,19 +92,21 @@ bool fp_segment_supported(const ProjGeom &g);
 unsigned fp_segment(FPSegment &sg, const void *vol, const ProjGeom &g, const float *axes, int nAxes,
                     float *casImgs, unsigned workStart, const unsigned *check = nullptr);
 hipError_t launch_forward_project_multi(const FPMultiArgs &m, hipStream_t s);
-// The fast back projection walks bricks in a centre-out order; these give the
-// table length (0 when the generic kernel is used) and fill it (host memory).
-int bp_brick_count(int V, bool fast);
-void bp_brick_order(int V, int *out);
+// The fast and the column kernels walk bricks of 8 x 8 x depth (8, or
+// col_depth) in a centre-out order; these give the table's length and
+// fill it (host memory).
+int bp_brick_count(int V, int depth);
+void bp_brick_order(int V, int depth, int *out);
 // True when launch_back_project takes the fast path for this geometry.
 bool bp_uses_fast_path(const ProjGeom &g);
 // Exact transpose of launch_forward_project (atomic scatter into volAcc).
 // With check pointing at launch_check_volume's flag for the nAxes * M * M CAS
 // image values and the table, the scatter skips the taps of weight 0 (same
-// sums, smaller boxes).
+// sums, smaller boxes).  With columns (launch_check_back's flag, after
+// launch_columns) it does what the columns leave.
 hipError_t launch_back_project_adjoint(float *volAcc, const ProjGeom &g, const float *axes,
                                        int nAxes, const float *casImgs, hipStream_t s,
-                                       const unsigned *check = nullptr);
+                                       const unsigned *check = nullptr, const unsigned *columns = nullptr);
 
 // ---- image chains (2-D, batched) ----------------------------------------
 // CAS images (n x M x M) -> Hermitian half spectra (n x M x (M/2+1)) ready for

@@ -21,7 +21,9 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
+#include <vector>
 
 namespace mgg {
 namespace {
@@ -144,6 +146,8 @@ struct FPArgs {
     unsigned perXcd, totalWork;
     int maskD2;  // fp_lds_kernel: largest integer d2 with sqrtf((float)d2) <= maskR (-1: none)
     const unsigned *check;  // fp_lds_kernel with the 501-entry table: launch_check_volume's flag, or null
+    const unsigned *columns;  // adj_lds_kernel: launch_check_back's flag when the column launches came first, or null
+    float orthTol;            // with columns: frames they took are orthonormal to this
 };
 
 constexpr int KFP_FAST = 501;  // the table the mixed-volume launch requires (kerScale 125, kerCenter 250)
@@ -779,9 +783,22 @@ __global__ __launch_bounds__(kThreads) void fp_lds_multi_kernel(FPMultiArgs m)
         a.maskR = 0.f; a.kerScale = 125.0f; a.kerCenter = 250.0f; a.fW = 2.0f;
         a.convW = 2; a.tilesPerRow = sg.tilesPerRow; a.tilesPerImg = sg.tilesPerImg;
         a.perXcd = 0; a.totalWork = 0; a.maskD2 = sg.maskD2; a.check = sg.check;
+        a.columns = nullptr; a.orthTol = 0.f;
         if (fp_win4(sg.check)) fp_lds_tile<DT, true, true, BIG>(a, nullptr, sbox[wv], work - sg.workStart, ln);
         else fp_lds_tile<DT, true, false, BIG>(a, nullptr, sbox[wv], work - sg.workStart, ln);
     }
+}
+
+// The transpose has no use for a direction's third vector: a9[6..8] = u x v,
+// true when [u v] is orthonormal to tol.
+__device__ __forceinline__ bool adj_plane(float (&a)[9], float tol)
+{
+    a[6] = a[1] * a[5] - a[2] * a[4];
+    a[7] = a[2] * a[3] - a[0] * a[5];
+    a[8] = a[0] * a[4] - a[1] * a[3];
+    return fabsf(a[0] * a[0] + a[1] * a[1] + a[2] * a[2] - 1.f) <= tol &&
+           fabsf(a[3] * a[3] + a[4] * a[4] + a[5] * a[5] - 1.f) <= tol &&
+           fabsf(a[0] * a[3] + a[1] * a[4] + a[2] * a[5]) <= tol;
 }
 
 // ---------------------------------------------------------------------------
@@ -804,7 +821,7 @@ __global__ __launch_bounds__(kThreads) void fp_lds_multi_kernel(FPMultiArgs m)
 template <bool FAST, bool W4>
 __device__ __forceinline__ void adj_lds_tile(const FPArgs &p, const float *__restrict__ sker,
                                              float *__restrict__ box, const float *__restrict__ img,
-                                             float *__restrict__ volAcc, unsigned work, int ln)
+                                             float *__restrict__ volAcc, unsigned work, int ln, bool skewOnly)
 {
     const int a = (int)(work / (unsigned)p.tilesPerImg);
     const int tile = (int)(work - (unsigned)a * (unsigned)p.tilesPerImg);
@@ -821,6 +838,10 @@ __device__ __forceinline__ void adj_lds_tile(const FPArgs &p, const float *__res
     const float *ax = p.axes + (size_t)9 * a;
     const float u0 = ax[0], u1 = ax[1], u2 = ax[2];
     const float v0 = ax[3], v1 = ax[4], v2 = ax[5];
+    if (skewOnly) {  // the column launches have done the orthonormal planes
+        float f[9] = {u0, u1, u2, v0, v1, v2, 0.f, 0.f, 0.f};
+        if (adj_plane(f, p.orthTol)) return;
+    }
     const float fi = (float)(i - ci), fj = (float)(j - ci);
     const float x = ref_sum2c(u0, fi, v0, fj, (float)cv);
     const float y = ref_sum2c(u1, fi, v1, fj, (float)cv);
@@ -999,17 +1020,21 @@ __global__ __launch_bounds__(kThreads) void adj_lds_kernel(FPArgs p, const float
 {
     __shared__ float sker[FPKER];
     __shared__ float sbox[4][FPBOX];
+    // What the column launches have left (launch_check_back's flag): all
+    // frames, those that are not orthonormal, or none.
+    const unsigned done = p.columns != nullptr ? (unsigned)__builtin_amdgcn_readfirstlane(*p.columns) : 0u;
+    if (done == 3u) return;
     if (!FAST) {
         for (int t = threadIdx.x; t < p.K; t += kThreads) sker[t] = p.ker[t];
         __syncthreads();
     }
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
-    if (FAST && fp_win4(p.check)) {
+    if (FAST && (done != 0u || fp_win4(p.check))) {
         for (unsigned work = blockIdx.x * 4u + (unsigned)wv; work < p.totalWork; work += gridDim.x * 4u)
-            adj_lds_tile<FAST, true>(p, sker, sbox[wv], img, volAcc, work, ln);
+            adj_lds_tile<FAST, true>(p, sker, sbox[wv], img, volAcc, work, ln, done != 0u);
     } else {
         for (unsigned work = blockIdx.x * 4u + (unsigned)wv; work < p.totalWork; work += gridDim.x * 4u)
-            adj_lds_tile<FAST, false>(p, sker, sbox[wv], img, volAcc, work, ln);
+            adj_lds_tile<FAST, false>(p, sker, sbox[wv], img, volAcc, work, ln, false);
     }
 }
 
@@ -1032,8 +1057,10 @@ struct BPArgs {
     int maskD2;  // largest integer d2 with sqrtf((float)d2) <= maskR (-1: none)
     int posRound;  // bp_fast_kernel: in-mask voxels of orthonormal frames project to fi, fj >= 0.5
     int maskLo;    // smallest coordinate of an in-mask voxel (V/2 - floor(sqrt(maskD2)))
-    const int *order;  // bp_fast_kernel: brick id per work item, heaviest first
+    const int *order;  // bp_fast_kernel, bp_col_kernel: brick id per work item, heaviest first
     unsigned perXcd, totalWork;
+    const unsigned *check;  // bp_fast_kernel: launch_check_back's flag, or null
+    float orthTol;          // frames that the column launches take are orthonormal to this
 };
 
 constexpr int BPX = 8, BPY = 8, BPZ = 4;
@@ -1256,17 +1283,30 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-template <bool DENS>
-__global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
+// [u v n] orthonormal to tol (false for non-finite frames).
+__device__ __forceinline__ bool bp_orthonormal(const float (&a)[9], float tol)
+{
+    const float uu = a[0] * a[0] + a[1] * a[1] + a[2] * a[2];
+    const float vv = a[3] * a[3] + a[4] * a[4] + a[5] * a[5];
+    const float nn = a[6] * a[6] + a[7] * a[7] + a[8] * a[8];
+    const float uv = a[0] * a[3] + a[1] * a[4] + a[2] * a[5];
+    const float un = a[0] * a[6] + a[1] * a[7] + a[2] * a[8];
+    const float vn = a[3] * a[6] + a[4] * a[7] + a[5] * a[8];
+    return fabsf(uu - 1.f) <= tol && fabsf(vv - 1.f) <= tol && fabsf(nn - 1.f) <= tol &&
+           fabsf(uv) <= tol && fabsf(un) <= tol && fabsf(vn) <= tol;
+}
+
+template <bool DENS, int BFW>
+__global__ __launch_bounds__(64 * BFW) void bp_fast_kernel(BPArgs p)
 {
     __shared__ float sker[KTOT];
     __shared__ float sax[BPCH * 9];
     __shared__ int sidx[BPCH];
-    __shared__ int swave[kThreads / 64];
-    __shared__ int snon[kThreads / 64];
-    __shared__ float sacc[4][BV];
-    __shared__ float sden[DENS ? 4 : 1][DENS ? BV : 1];
-    __shared__ unsigned short squeue[4][QCAP];
+    __shared__ int swave[BFW];
+    __shared__ int snon[BFW];
+    __shared__ float sacc[BFW][BV];
+    __shared__ float sden[DENS ? BFW : 1][DENS ? BV : 1];
+    __shared__ unsigned short squeue[BFW][QCAP];
 
     // Bricks near the centre meet every direction and bricks near the mask edge
     // few, so the order table puts the heavy (central) bricks first and
@@ -1284,9 +1324,13 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
         float dz = fmaxf(fmaxf((float)(oz - cv), (float)(cv - (oz + BB - 1))), 0.f);
         if (dx * dx + dy * dy + dz * dz > (p.maskR + 1.f) * (p.maskR + 1.f)) return;
     }
+    // What the column launches have left: everything, the frames that are not
+    // orthonormal, or nothing.
+    const unsigned done = p.check != nullptr ? (unsigned)__builtin_amdgcn_readfirstlane(*p.check) : 0u;
+    if (done == 3u) return;
     const int t = threadIdx.x;
-    for (int k = t; k < KTOT; k += kThreads) sker[k] = p.ker[min(max(k - KPAD, 0), KFAST - 1)];
-    for (int k = t; k < 4 * BV; k += kThreads) {
+    for (int k = t; k < KTOT; k += (64 * BFW)) sker[k] = p.ker[min(max(k - KPAD, 0), KFAST - 1)];
+    for (int k = t; k < BFW * BV; k += (64 * BFW)) {
         (&sacc[0][0])[k] = 0.f;
         if (DENS) (&sden[0][0])[k] = 0.f;
     }
@@ -1326,15 +1370,9 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
             const float d = bcx * a9[6] + bcy * a9[7] + bcz * a9[8];
             const float sup = bc * (fabsf(a9[6]) + fabsf(a9[7]) + fabsf(a9[8]));
             pass = fabsf(d) <= p.hw + sup + 1e-3f;
-            // [u v n] orthonormal to 1e-4 (rotation matrices are, to ~1e-7)
-            const float uu = a9[0] * a9[0] + a9[1] * a9[1] + a9[2] * a9[2];
-            const float vv = a9[3] * a9[3] + a9[4] * a9[4] + a9[5] * a9[5];
-            const float nn = a9[6] * a9[6] + a9[7] * a9[7] + a9[8] * a9[8];
-            const float uv = a9[0] * a9[3] + a9[1] * a9[4] + a9[2] * a9[5];
-            const float un = a9[0] * a9[6] + a9[1] * a9[7] + a9[2] * a9[8];
-            const float vn = a9[3] * a9[6] + a9[4] * a9[7] + a9[5] * a9[8];
-            orth = fabsf(uu - 1.f) <= 1e-4f && fabsf(vv - 1.f) <= 1e-4f && fabsf(nn - 1.f) <= 1e-4f &&
-                   fabsf(uv) <= 1e-4f && fabsf(un) <= 1e-4f && fabsf(vn) <= 1e-4f;
+            // rotation matrices are orthonormal to ~1e-7
+            orth = bp_orthonormal(a9, 1e-4f);
+            if (done != 0u && bp_orthonormal(a9, p.orthTol)) pass = false;
         }
         const unsigned long long bal = __ballot(pass);
         const unsigned long long nonOrth = __ballot(!orth);
@@ -1343,10 +1381,13 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
             snon[wv] = nonOrth != 0ull;
         }
         __syncthreads();
-        const bool chunkOrtho = !(snon[0] | snon[1] | snon[2] | snon[3]);
+        int non = 0;
+#pragma unroll
+        for (int w = 0; w < BFW; w++) non |= snon[w];
+        const bool chunkOrtho = non == 0;
         int off = 0, total = 0;
 #pragma unroll
-        for (int w = 0; w < kThreads / 64; w++) {
+        for (int w = 0; w < BFW; w++) {
             off += (w < wv) ? swave[w] : 0;
             total += swave[w];
         }
@@ -1362,7 +1403,7 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
         // Their active voxels stream through the wave's FIFO queue; every
         // full group of 64 entries is gathered with all lanes busy.
         int head = 0, tail = 0;  // queue indices (uniform), ring of size QCAP
-        for (int q = wv; q < total || tail > head; q += 4) {
+        for (int q = wv; q < total || tail > head; q += BFW) {
             if (q < total) {
                 const float *ax = sax + q * 9;
                 const float n0 = ax[6], n1 = ax[7], n2 = ax[8];
@@ -1382,7 +1423,7 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
                     tail += __popcll(b);
                 }
             }
-            const bool last = q + 4 >= total;
+            const bool last = q + BFW >= total;
             wave_lds_sync();
             // Gather full groups (and, after the last direction, the rest).
             auto gather = [&](auto formT) {
@@ -1499,7 +1540,7 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
         }
     }
     __syncthreads();
-    for (int k = t; k < BV; k += kThreads) {
+    for (int k = t; k < BV; k += (64 * BFW)) {
         const int lx = k & 7, ly = (k >> 3) & 7, lz = k >> 6;
         const int vi = ox + lx, vj = oy + ly, vk = oz + lz;
         if (vi >= V || vj >= V || vk >= V) continue;
@@ -1508,14 +1549,445 @@ __global__ __launch_bounds__(kThreads) void bp_fast_kernel(BPArgs p)
         const size_t vidx = ((size_t)vk * V + vj) * V + vi;
         double s = (double)p.vol[vidx];
 #pragma unroll
-        for (int w = 0; w < 4; w++) s += (double)sacc[w][k];
+        for (int w = 0; w < BFW; w++) s += (double)sacc[w][k];
         p.vol[vidx] = (float)s;
         if (DENS) {
             double d = (double)p.dens[vidx];
 #pragma unroll
-            for (int w = 0; w < 4; w++) d += (double)sden[w][k];
+            for (int w = 0; w < BFW; w++) d += (double)sden[w][k];
             p.dens[vidx] = (float)d;
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Back projection, and the forward gather's exact transpose, by voxel columns:
+// the path of orthonormal frames whose CAS images are finite (launch_check_back's
+// flag; bp_fast_kernel or adj_lds_kernel runs what is left).
+//
+// bp_fast_kernel looks up three table entries for each of the 25 pixels of
+// each voxel.  But a pixel's position does not depend on the voxel, and along
+// the axis c on which the direction's normal is largest the plane's slab holds
+// 4 to 7 consecutive voxels of a column.  So a lane owns a column and visits
+// each pixel that can reach any of these voxels once: one position, one lookup
+// for each of the two cross axes (shared by the column), and one index for all
+// voxels of the column, whose entries lie 125 apart: the LDS table holds pairs
+// (T[k], T[k - 125]), zero outside the table, and entry pairs 250 apart give
+// the K weights in (K + 1) / 2 reads (a random 8-byte read costs what a 4-byte
+// one does: 2.8 against 2.6 ns per wave and CU).  Per unit of slab area about
+// 27 pixels are visited instead of 4 x 25 taps.  The transpose is the same
+// gather with the windows' other bounds (|z - p_c| < 2 instead of the slab, no
+// 5 x 5 windows, the mask on the pixels), where adj_lds_kernel spends half its
+// time in 10 global atomics per pixel; its sums come in a fixed order.
+//
+// Work layout.  A wave owns 8 x 8 columns, bc_depth voxels long; the waves of
+// a workgroup share them and take every fourth (eighth) direction each, into
+// LDS accumulators of their own (lane-private columns: plain adds, no bank
+// conflicts), combined in FP64 at the end.  The axis of the columns is that of
+// the launch: three launches, one after the other, each taking the directions
+// of its axis.  A wave handles one direction at a time, so the list of pixel
+// offsets (from the pixel nearest to where the column meets the plane) is wave
+// uniform and its position arithmetic reads the frame from scalar registers.
+// The list holds every offset that can reach weight != 0 for some position of
+// the crossing point inside its pixel: |u_a i + v_a j| <= 2 + (|u_a| + |v_a|) / 2
+// for both cross axes a.
+//
+// Decisions are the reference's, each in its own FP32 arithmetic: the slab
+// test, the rounded centre of every voxel's 5 x 5 window (a bit mask over the
+// offsets per voxel) and the table indices.  The cross axes use kb_form's
+// fused index (BP_FORM_A_MIN).  Along the column, slot k's index is slot 0's
+// minus 125 k unless the FP32 rounding of the larger index value crosses a
+// half-integer that the smaller one does not; then the larger one is exactly a
+// half-integer (its spacing is at least the smaller one's and both are the
+// same distance from theirs), so lanes that meet one take each slot's index by
+// itself.
+//
+// Measured: 2,000 directions at N=128 6.9 (bp_fast_kernel) -> 6.35 ms, 1,000 at
+// N=96 3.0 -> 2.0 ms; the transpose of 2,048 at N=96 6.5 -> 5.6 ms.  Bound by
+// issue and LDS together: a pixel takes 37 vector instructions and five random
+// table reads (13.6 ns per wave and CU of the 14.6 measured), and another 40%
+// of the time goes to per-row and per-column work (windows, row bounds) at
+// four waves per SIMD.  Blocks of 32 voxels (three waves per SIMD) ran 6.8 ms,
+// four pixels at a time 7.0, one row buffer of three pixels with a compact
+// loop 7.4.
+// ---------------------------------------------------------------------------
+constexpr int BCN = 8;                        // columns per block edge
+enum : int { COL_BACK = 0, COL_ADJOINT = 1 };
+// Index range of the pair table (swept over 200,000 frames, half of them with
+// the normal near a diagonal: -566 to 1,189 for columns of up to six slab
+// voxels, -787 to 1,401 for up to ten transposed ones).
+constexpr int ct_lo(int mode) { return mode == COL_BACK ? -576 : -800; }
+constexpr int ct_hi(int mode) { return mode == COL_BACK ? 1200 : 1416; }
+// Voxels of a block along its columns: four (transpose: three) workgroups of
+// four waves per CU.
+constexpr int bc_depth(int mode) { return mode == COL_BACK ? 24 : 32; }
+
+struct BPColArgs {
+    BPArgs b;
+    int blocks8;       // blocks along a cross axis
+    int reachD2;       // largest squared distance from the centre of a voxel that is given values
+};
+
+__device__ __forceinline__ float read_lane_f(float x, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+
+template <int MODE>
+__device__ __forceinline__ float2 ct_pair(const float2 *__restrict__ st, int idx) { return st[idx - ct_lo(MODE)]; }
+
+// One direction's visit of a wave's 64 columns, K slots per column.
+// A: column axis (0, 1, 2 = x, y, z); the cross axes a, b are the others in
+// order.  Vectors are in (a, b, c) order; onbits: slots that are active voxels;
+// v0: first slot's coordinate along c.
+
+template <int A, int K, int MODE>
+struct ColVisit {
+    static constexpr bool GATE = MODE == COL_BACK;
+    // Back projection looks up p - v, the forward gather and so its transpose
+    // v - p (a half-integer index rounds the other way).  The slots go along c
+    // so that slot 0 has the largest index: up, or down.
+    static constexpr int SG = GATE ? 1 : -1;
+    static constexpr float SC = GATE ? 125.0f : -125.0f;
+
+    static __device__ __forceinline__ float coord(float da, float db, float dc, float qa, float qb, float qc)
+    {
+        // ref_sum3 in x, y, z order
+        if constexpr (A == 2) return ref_sum3(da, qa, db, qb, dc, qc);
+        else if constexpr (A == 1) return ref_sum3(da, qa, dc, qc, db, qb);
+        else return ref_sum3(dc, qc, da, qa, db, qb);
+    }
+
+    // half: half the extent along c of the voxels a column can be given values
+    // in, from where it meets the plane.
+    static __device__ __forceinline__ void run(
+        const float2 *__restrict__ st, float *__restrict__ acc, const float *__restrict__ im,
+        int M, int cv, int maskD2, int ln, float da, float db, int dzMax, int oc, int depth, int depthMax, float hw,
+        float half, float ua, float ub, float uc, float va, float vb, float vc, float na, float nb, float nc)
+    {
+        const int ci = M / 2, M2 = M * M;
+        const float cvf = (float)cv, cif = (float)ci;
+        // where the column meets the plane, and its first voxel
+        const float inv = __builtin_amdgcn_rcpf(nc);
+        const float zc = -(na * da + nb * db) * inv;
+        // relative to the volume's centre
+        const int v0 = GATE ? (int)ceilf(zc - half - 5e-3f) : (int)floorf(zc + half + 5e-3f);
+        const float fic = ua * da + ub * db + uc * zc, fjc = va * da + vb * db + vc * zc;
+        int I0 = (int)rintf(fic), J0 = (int)rintf(fjc);
+
+        unsigned onbits = 0;
+        unsigned win[GATE ? K : 1];  // voxel k's 5 x 5 window: bits 8 + di low half, 8 + dj high half
+        const int si0 = ci + I0 - 6, sj0 = ci + J0 - 22;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int dz = v0 + SG * k;
+            bool on = (unsigned)(dz + cv - oc) < (unsigned)depth;
+            if constexpr (GATE) {
+                const float dc = (float)v0 + (float)k;
+                const float fk = coord(da, db, dc, na, nb, nc);
+                on = on && fabsf(fk) <= hw && abs(dz) <= dzMax;
+                const float fi = coord(da, db, dc, ua, ub, uc) + cif;
+                const float fj = coord(da, db, dc, va, vb, vc) + cif;
+                // the window's centre is at most 3 pixels from (I0, J0) for
+                // the slab's voxels
+                const unsigned w = (0x1Fu << ((cvt_rpi(fi) - si0) & 31)) | (0x1Fu << ((cvt_rpi(fj) - sj0) & 31));
+                win[k] = on ? w : 0u;
+            }
+            onbits |= on ? (1u << k) : 0u;
+        }
+        // Pixels that a column visits are within 9 of (I0, J0) in each index.
+        const int ai = abs(I0), aj = abs(J0);
+        if (!GATE && (dzMax < 0 || max(ai - 9, 0) * max(ai - 9, 0) + max(aj - 9, 0) * max(aj - 9, 0) > maskD2)) onbits = 0;
+        const bool live = onbits != 0u;
+        if (__ballot(live) == 0ull) return;
+        // a column without a voxel to fill idles on the centre's
+        const float ea = live ? da : 0.f, eb = live ? db : 0.f;
+        const int e0c = live ? v0 : GATE ? (int)ceilf(-half - 5e-3f) : (int)floorf(half + 5e-3f);
+        if (!live) I0 = J0 = 0;
+
+        // Pixel offsets: lane r < 16 bounds row dj = r - 8 (rows with pixels are
+        // consecutive).
+        float rowLo = -8.f;
+        int rowCnt;
+        {
+            const float dj = (float)((ln & 15) - 8);
+            float hi = 7.f;
+            auto bound = [&](float u, float v) {
+                const float L = 2.02f + 0.5f * (fabsf(u) + fabsf(v));
+                if (fabsf(u) < 1e-6f) {
+                    if (fabsf(v * dj) > L) hi = -9.f;
+                } else {
+                    const float r = __builtin_amdgcn_rcpf(u), p = (-L - v * dj) * r, q = (L - v * dj) * r;
+                    rowLo = fmaxf(rowLo, ceilf(fminf(p, q)));
+                    hi = fminf(hi, floorf(fmaxf(p, q)));
+                }
+            };
+            bound(ua, va);
+            bound(ub, vb);
+            rowCnt = max((int)(hi - rowLo) + 1, 0);
+        }
+        const unsigned rows = (unsigned)__ballot(rowCnt > 0 && ln < 16);
+        if (rows == 0u) return;
+        int r = __builtin_ctz(rows);
+        const int rEnd = 32 - __builtin_clz(rows);
+
+        // index constants 250 -+ 125 v of the column and of its first slot
+        const float cA = fmaf(-SC, ea + cvf, 250.0f), cB = fmaf(-SC, eb + cvf, 250.0f);
+        const float cC = fmaf(-SC, (float)(e0c + cv), 250.0f);
+        const int lin0 = (J0 + ci) * M + (I0 + ci);
+        // every pixel of every lane is in the image (BACK) or the mask (ADJOINT)
+        const bool allIn = GATE ? __all(lin0 >= 8 * M + 8 && lin0 + 8 * M + 14 <= M2)
+                                : __all(!live || ((ai + 14) * (ai + 14) + (aj + 9) * (aj + 9) <= maskD2 &&
+                                                  (ai + 14) * (ai + 14) <= maskD2));
+        const float I0f = (float)I0;
+        float djf = (float)(J0 + r - 8);
+
+        float s[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) s[k] = 0.f;
+
+        // The values of six consecutive pixels from offset off (a row has five
+        // on average).
+        auto load = [&](int off, int row, int di, float (&x)[6]) {
+            if (allIn) {
+                const float *ip = (const float *)((const char *)(im + off) + (unsigned)lin0 * 4u);
+                f4 q;
+                __builtin_memcpy(&q, ip, 16);
+                x[0] = q.x; x[1] = q.y; x[2] = q.z; x[3] = q.w;
+                __builtin_memcpy(&x[4], ip + 4, 8);
+            } else {
+                // The reference's back projection bounds only the linear index
+                // (gpuBackProject.cu:99): windows wrap across rows.  The
+                // forward projection writes the pixels of the mask disc.
+                const int dj = J0 + row - 8;
+#pragma unroll
+                for (int e = 0; e < 6; e++) {
+                    const int lin = lin0 + off + e, i = I0 + di + e;
+                    const bool ok = GATE ? lin >= 0 && lin < M2
+                                         : i * i + dj * dj <= maskD2 && (unsigned)(i + ci) < (unsigned)M &&
+                                               (unsigned)(dj + ci) < (unsigned)M;
+                    const float raw = im[min(max(lin, 0), M2 - 1)];
+                    x[e] = ok ? raw : 0.f;
+                }
+            }
+        };
+        // only the longest columns reach past the table's ends
+        constexpr bool LONG = GATE ? K == 7 : K > 10;
+        auto clampC = [](int i) { return LONG ? min(max(i, ct_lo(MODE)), ct_hi(MODE) - 1) : i; };
+        float Ba, Bb, Bc;
+        unsigned eff[GATE ? K : 1];
+        // NP pixels of the current row from offset di on (bit di + 8 of eff).
+        auto pixels = [&](float Df, int di, const float *val, auto np) {
+            constexpr int NP = decltype(np)::value;
+            float wab[NP];
+            float2 wc[NP][(K + 1) / 2];
+            float sc[NP], pc[NP];
+            bool tie = false;
+#pragma unroll
+            for (int q = 0; q < NP; q++) {
+                const float Di = Df + (float)q;
+                const float pa = fmaf(Di, ua, Ba) + cvf, pb = fmaf(Di, ub, Bb) + cvf;
+                pc[q] = fmaf(Di, uc, Bc) + cvf;
+                sc[q] = fmaf(pc[q], SC, cC);
+                tie = tie || __builtin_amdgcn_fractf(sc[q]) == 0.5f;
+                const int ic = cvt_rpi(sc[q]);
+                wab[q] = ct_pair<MODE>(st, cvt_rpi(fmaf(pa, SC, cA))).x * ct_pair<MODE>(st, cvt_rpi(fmaf(pb, SC, cB))).x;
+#pragma unroll
+                for (int h = 0; h < (K + 1) / 2; h++) wc[q][h] = ct_pair<MODE>(st, clampC(ic - 250 * h));
+            }
+            if (__any(tie)) {
+#pragma unroll
+                for (int q = 0; q < NP; q++)
+#pragma unroll
+                    for (int k = 0; k < K; k++) {
+                        float w = ct_pair<MODE>(st, clampC(cvt_rpi(fmaf(pc[q], SC, cC - 125.0f * k)))).x;
+                        // keeps these loads apart from the paired ones (the
+                        // compiler merges both into K single loads)
+                        __asm__ volatile("" : "+v"(w));
+                        if (k & 1) wc[q][k / 2].y = w; else wc[q][k / 2].x = w;
+                    }
+            }
+#pragma unroll
+            for (int q = 0; q < NP; q++) {
+                const float wv = wab[q] * val[q];
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    float w = (k & 1) ? wc[q][k / 2].y : wc[q][k / 2].x;
+                    if constexpr (GATE)
+                        w = __int_as_float(__float_as_int(w) & __builtin_amdgcn_sbfe((int)eff[k], di + 8 + q, 1));
+                    s[k] = fmaf(wv, w, s[k]);
+                }
+            }
+        };
+        using One = std::integral_constant<int, 1>;
+        using Two = std::integral_constant<int, 2>;
+        using Three = std::integral_constant<int, 3>;
+        // The next row's first six values are loaded while a row is gathered.
+        float val[6];
+        float lo = read_lane_f(rowLo, r);
+        int cnt = __builtin_amdgcn_readlane(rowCnt, r), off = (r - 8) * M + (int)lo;
+        load(off, r, (int)lo, val);
+        while (true) {
+            const float loN = read_lane_f(rowLo, r + 1);
+            const int cntN = __builtin_amdgcn_readlane(rowCnt, r + 1), offN = (r - 7) * M + (int)loN;
+            float nval[6];
+            if (r + 1 < rEnd) load(offN, r + 1, (int)loN, nval);
+            Ba = djf * va; Bb = djf * vb; Bc = djf * vc;
+#pragma unroll
+            for (int k = 0; k < (GATE ? K : 0); k++)
+                eff[k] = win[k] & (unsigned)__builtin_amdgcn_sbfe((int)win[k], r + 16, 1);
+            const float Df = I0f + lo;
+            const int di = (int)lo;
+            if (cnt >= 3) pixels(Df, di, val, Three{});
+            else if (cnt == 2) pixels(Df, di, val, Two{});
+            else if (cnt == 1) pixels(Df, di, val, One{});
+            if (cnt >= 6) pixels(Df + 3.f, di + 3, val + 3, Three{});
+            else if (cnt == 5) pixels(Df + 3.f, di + 3, val + 3, Two{});
+            else if (cnt == 4) pixels(Df + 3.f, di + 3, val + 3, One{});
+            if (cnt > 6) {
+                for (int e = 6; e < cnt; e += 2) {  // one past the row's end weighs 0
+                    float xv[6];
+                    load(off + e, r, di + e, xv);
+                    pixels(Df + (float)e, di + e, xv, Two{});
+                }
+            }
+            if (++r >= rEnd) break;
+            lo = loN; cnt = cntN; off = offN;
+            djf += 1.f;
+#pragma unroll
+            for (int e = 0; e < 6; e++) val[e] = nval[e];
+        }
+        // Slots that are no active voxel go to the accumulators' spare row.
+        int row[K];
+        float ov[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            row[k] = ((onbits >> k) & 1u ? v0 + SG * k + cv - oc : depthMax) * 64 + ln;
+            ov[k] = acc[row[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) acc[row[k]] = ov[k] + s[k];
+        __asm__ volatile("" ::: "memory");
+    }
+};
+
+template <int A, int MODE, int BCW>
+__global__ __launch_bounds__(64 * BCW, MODE == COL_BACK ? 4 : 3) void col_kernel(BPColArgs p)
+{
+    constexpr bool GATE = MODE == COL_BACK;
+    constexpr int D = bc_depth(MODE), LO = ct_lo(MODE), NT = ct_hi(MODE) - LO;
+    __shared__ float2 st[NT];
+    __shared__ float sacc[BCW][64 * (D + 1)];  // and a spare row
+
+    // not set: the voxel (tile) kernel does it all
+    if ((__builtin_amdgcn_readfirstlane(*p.b.check) & 1u) == 0u) return;
+    const unsigned work = (unsigned)p.b.order[blockIdx.x];
+    // block lattice (a, b, c), a fastest
+    const int bc = (int)(work / (unsigned)(p.blocks8 * p.blocks8));
+    const int rem = (int)(work - (unsigned)bc * (unsigned)(p.blocks8 * p.blocks8));
+    const int bb = rem / p.blocks8, ba = rem - bb * p.blocks8;
+    const int oa = ba * BCN, ob = bb * BCN, oc = bc * D;
+    const int V = p.b.V, M = p.b.M, cv = V / 2;
+    // Voxels farther from the centre than the mask radius (the transpose's
+    // windows: 2 sqrt(3) more) take nothing.
+    {
+        auto gap = [&](int o, int e) { return max(max(o - cv, cv - (o + e - 1)), 0); };
+        const int ga = gap(oa, BCN), gb = gap(ob, BCN), gc = gap(oc, D);
+        if (ga * ga + gb * gb + gc * gc > p.reachD2) return;
+    }
+    const int t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63;
+    for (int e = t; e < NT; e += 64 * BCW) {
+        const int i = e + LO, j = i - 125;
+        st[e] = make_float2(i >= 0 && i < KFAST ? p.b.ker[min(max(i, 0), KFAST - 1)] : 0.f,
+                            j >= 0 && j < KFAST ? p.b.ker[min(max(j, 0), KFAST - 1)] : 0.f);
+    }
+    for (int e = t; e < BCW * 64 * (D + 1); e += 64 * BCW) (&sacc[0][0])[e] = 0.f;
+    __syncthreads();
+
+    const int depth = min(D, V - oc);
+    // This lane's column, relative to the volume's centre, and how far the
+    // mask sphere (the volume) reaches along it (-1: not at all).
+    const int la = oa + (ln & 7) - cv, lb = ob + (ln >> 3) - cv;
+    int dzMax = -1;
+    if (oa + (ln & 7) < V && ob + (ln >> 3) < V) {
+        const int rest = p.b.maskD2 - la * la - lb * lb;
+        if (!GATE) {
+            dzMax = V;
+        } else if (rest >= 0) {
+            dzMax = (int)sqrtf((float)rest);
+            while (dzMax * dzMax > rest) dzMax--;
+            while ((dzMax + 1) * (dzMax + 1) <= rest) dzMax++;
+        }
+    }
+    const float da = (float)la, db = (float)lb;
+    const float mA = (float)(oa - cv) + 0.5f * (BCN - 1), mB = (float)(ob - cv) + 0.5f * (BCN - 1);
+    const float mC = (float)(oc - cv) + 0.5f * (D - 1);
+    constexpr int ia = A == 0 ? 1 : 0, ib = A == 2 ? 1 : 2, ic = A;
+
+    for (int base = 0; base < p.b.nAxes; base += BCW * 64) {
+        const int mine = base + BCW * ln + wv;
+        float a9[9];
+        bool pass = false;
+        if (mine < p.b.nAxes) {
+            const float *ax = p.b.axes + (size_t)9 * mine;
+#pragma unroll
+            for (int k = 0; k < 9; k++) a9[k] = ax[k];
+            const bool orth = GATE ? bp_orthonormal(a9, p.b.orthTol) : adj_plane(a9, p.b.orthTol);
+            const float n0 = fabsf(a9[6 + ia]), n1 = fabsf(a9[6 + ib]), n2 = fabsf(a9[6 + ic]);
+            // the launch whose axis is the normal's largest (the first of equals)
+            const bool axis = (A == 0 ? n2 >= n0 : n2 > n0) && (A == 2 ? n2 > n1 : n2 >= n1);
+            const float dist = mA * a9[6 + ia] + mB * a9[6 + ib] + mC * a9[6 + ic];
+            const float reach = GATE ? p.b.hw : 2.f * (n0 + n1 + n2);  // a slab, or cubes of half edge 2
+            pass = axis && orth && fabsf(dist) <= reach + 0.5f * (BCN - 1) * (n0 + n1) + 0.5f * (D - 1) * n2 + 1e-2f;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 9; k++) a9[k] = 0.f;
+        }
+        for (unsigned long long todo = __ballot(pass); todo != 0ull; todo &= todo - 1ull) {
+            const int l = __builtin_ctzll(todo);
+            const float ua = read_lane_f(a9[ia], l), ub = read_lane_f(a9[ib], l), uc = read_lane_f(a9[ic], l);
+            const float va = read_lane_f(a9[3 + ia], l), vb = read_lane_f(a9[3 + ib], l), vc = read_lane_f(a9[3 + ic], l);
+            const float na = read_lane_f(a9[6 + ia], l), nb = read_lane_f(a9[6 + ib], l), nc = read_lane_f(a9[6 + ic], l);
+            const float *im = p.b.img + (size_t)(base + BCW * l + wv) * M * M;
+            // A column's voxels: |fk| <= 2, or (transpose) |z - p_c| < 2 of a
+            // pixel with |p_a - x_a|, |p_b - x_b| < 2: at most
+            // floor(2 half) + 1 consecutive ones.
+            const float half = (GATE ? p.b.hw : 2.f * (fabsf(na) + fabsf(nb) + fabsf(nc))) *
+                               __builtin_amdgcn_rcpf(fabsf(nc));
+            const float len = 2.f * half + 1.5e-2f;
+#define MGG_VISIT(KS) ColVisit<A, KS, MODE>::run(st, sacc[wv], im, M, cv, p.b.maskD2, ln, da, \
+                                                       db, dzMax, oc, depth, D, p.b.hw, half, ua, ub, uc, va, vb, \
+                                                       vc, na, nb, nc)
+            if constexpr (GATE) {
+                if (__builtin_amdgcn_readfirstlane(len < 5.f)) MGG_VISIT(5);
+                else if (__builtin_amdgcn_readfirstlane(len < 6.f)) MGG_VISIT(6);
+                else MGG_VISIT(7);
+            } else {
+                if (__builtin_amdgcn_readfirstlane(len < 6.f)) MGG_VISIT(6);
+                else if (__builtin_amdgcn_readfirstlane(len < 8.f)) MGG_VISIT(8);
+                else if (__builtin_amdgcn_readfirstlane(len < 10.f)) MGG_VISIT(10);
+                else MGG_VISIT(14);
+            }
+#undef MGG_VISIT
+        }
+    }
+    __syncthreads();
+    // Add to the volume, x fastest: the columns' layout is [c][b][a].
+    for (int e = t; e < 64 * D; e += 64 * BCW) {
+        int qa, qb, qc;
+        if (A == 0) { qc = e % D; qa = (e / D) & 7; qb = e / (8 * D); }
+        else { qa = e & 7; qb = (e >> 3) & 7; qc = e >> 6; }
+        const int xa = oa + qa, xb = ob + qb, xc = oc + qc;
+        if (xa >= V || xb >= V || xc >= V) continue;
+        const int d2 = (xa - cv) * (xa - cv) + (xb - cv) * (xb - cv) + (xc - cv) * (xc - cv);
+        if (d2 > p.reachD2) continue;
+        const int x = A == 0 ? xc : xa, y = A == 0 ? xa : A == 1 ? xc : xb, z = A == 2 ? xc : xb;
+        const size_t vidx = ((size_t)z * V + y) * V + x;
+        const int slot = qc * 64 + qb * 8 + qa;
+        double sum = (double)p.b.vol[vidx];
+#pragma unroll
+        for (int w = 0; w < BCW; w++) sum += (double)sacc[w][slot];
+        p.b.vol[vidx] = (float)sum;
     }
 }
 
@@ -2382,40 +2854,76 @@ __global__ void k_fill(float *__restrict__ p, float v, size_t n)
 // the table's verdict, then k_check_volume clears it on any non-finite voxel
 // (all finding workgroups store the same 0).
 // ---------------------------------------------------------------------------
-__global__ void k_check_table(const float *__restrict__ ker, int K, unsigned *__restrict__ check)
+__global__ void k_check_table(const float *__restrict__ ker, int K, unsigned *__restrict__ check, unsigned good)
 {
     bool ok = true;
     for (int t = threadIdx.x; t < K; t += blockDim.x) ok = ok && __builtin_isfinite(ker[t]);
     ok = __syncthreads_and(ok);
-    if (threadIdx.x == 0) *check = (ok && K == KFP_FAST && ker[0] == 0.f && ker[K - 1] == 0.f) ? 1u : 0u;
+    if (threadIdx.x == 0) *check = (ok && K == KFP_FAST && ker[0] == 0.f && ker[K - 1] == 0.f) ? good : 0u;
 }
 
 // Non-finite = exponent field all ones (FP32 0x7f800000, BF16 0x7f80, FP16 0x7c00).
-template <int DT>
-__global__ void k_check_volume(const void *__restrict__ vol, size_t n, unsigned *__restrict__ check)
+// The calling thread's share of n FP32 values.
+__device__ __forceinline__ bool any_nonfinite(const unsigned *__restrict__ w, size_t n)
 {
     const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, st = (size_t)gridDim.x * blockDim.x;
     bool bad = false;
-    if (DT == DT_F32) {
-        const unsigned *w = (const unsigned *)vol;
-        size_t e0 = 0;
-        if (((uintptr_t)w & 15u) == 0) {  // 16-byte loads over the aligned body
-            const size_t n4 = n / 4;
-            const u4 *w4 = (const u4 *)w;
-            for (size_t e = t0; e < n4; e += st) {
-                const u4 q = w4[e];
-                bad |= ((q.x & 0x7f800000u) == 0x7f800000u) | ((q.y & 0x7f800000u) == 0x7f800000u) |
-                       ((q.z & 0x7f800000u) == 0x7f800000u) | ((q.w & 0x7f800000u) == 0x7f800000u);
-            }
-            e0 = n4 * 4;
+    size_t e0 = 0;
+    if (((uintptr_t)w & 15u) == 0) {  // 16-byte loads over the aligned body
+        const size_t n4 = n / 4;
+        const u4 *w4 = (const u4 *)w;
+        for (size_t e = t0; e < n4; e += st) {
+            const u4 q = w4[e];
+            bad |= ((q.x & 0x7f800000u) == 0x7f800000u) | ((q.y & 0x7f800000u) == 0x7f800000u) |
+                   ((q.z & 0x7f800000u) == 0x7f800000u) | ((q.w & 0x7f800000u) == 0x7f800000u);
         }
-        for (size_t e = e0 + t0; e < n; e += st) bad |= (w[e] & 0x7f800000u) == 0x7f800000u;
+        e0 = n4 * 4;
+    }
+    for (size_t e = e0 + t0; e < n; e += st) bad |= (w[e] & 0x7f800000u) == 0x7f800000u;
+    return bad;
+}
+
+template <int DT>
+__global__ void k_check_volume(const void *__restrict__ vol, size_t n, unsigned *__restrict__ check)
+{
+    bool bad = false;
+    if (DT == DT_F32) {
+        bad = any_nonfinite((const unsigned *)vol, n);
     } else {
+        const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, st = (size_t)gridDim.x * blockDim.x;
         const uint16_t *h = (const uint16_t *)vol;
         const unsigned m = DT == DT_BF16 ? 0x7f80u : 0x7c00u;
         for (size_t e = t0; e < n; e += st) bad |= ((unsigned)h[e] & m) == m;
     }
     if (__syncthreads_or(bad) && threadIdx.x == 0) *check = 0u;
+}
+
+// *check = 3 where another flag says that table and images are finite.
+__global__ void k_check_from(const unsigned *__restrict__ finite, unsigned *__restrict__ check)
+{
+    *check = *finite == 1u ? 3u : 0u;
+}
+
+// The check behind the column kernels: k_check_table has set *check
+// to 3 or 0; a non-finite image value clears both bits (everything is left to
+// the other kernel), a frame that is not orthonormal to tol the second (that
+// frame is; planes: only [u v] counts).
+__global__ void k_check_back(const float *__restrict__ img, size_t n, const float *__restrict__ axes, int nAxes,
+                             float tol, int planes, unsigned *__restrict__ check)
+{
+    const bool bad = any_nonfinite((const unsigned *)img, n);
+    bool skew = false;
+    for (int a = blockIdx.x * blockDim.x + threadIdx.x; a < nAxes; a += gridDim.x * blockDim.x) {
+        float a9[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) a9[k] = axes[(size_t)9 * a + k];
+        skew = skew || !(planes ? adj_plane(a9, tol) : bp_orthonormal(a9, tol));
+    }
+    const bool anyBad = __syncthreads_or(bad), anySkew = __syncthreads_or(skew);
+    if (threadIdx.x == 0) {
+        if (anyBad) atomicAnd(check, 0u);
+        else if (anySkew) atomicAnd(check, 1u);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2636,6 +3144,7 @@ hipError_t launch_forward_project(const void *vol, int dtype, const ProjGeom &g,
     if (nAxes <= 0) return hipSuccess;
     FPArgs a;
     a.vol = vol; a.axes = axes; a.out = casImgs; a.ker = g.ker; a.check = nullptr;
+    a.columns = nullptr; a.orthTol = 0.f;
     a.V = g.V; a.M = g.M; a.K = g.K; a.nAxes = nAxes;
     a.maskR = ref_mask_radius(g.maskRadius);
     proj_consts(g, a.kerScale, a.kerCenter, a.fW, a.convW);
@@ -2743,41 +3252,70 @@ bool bp_uses_fast_path(const ProjGeom &g)
     return convW == 2 && kerScale == 125.0f && kerCenter == 250.0f && g.K == KFAST && g.V <= 8192;
 }
 
-int bp_brick_count(int V, bool fast)
+int bp_brick_count(int V, int depth)
 {
-    const int b = fast ? (V + BB - 1) / BB : 0;
-    return b * b * b;
+    const int b = (V + BB - 1) / BB;
+    return b * b * ((V + depth - 1) / depth);
 }
 
-void bp_brick_order(int V, int *out)
+void bp_brick_order(int V, int depth, int *out)
 {
-    // Bricks of edge BB sorted by the distance of their centre from the volume
-    // centre (ties by index): central bricks, which every direction's slab
-    // crosses, are dispatched first.
-    const int nb = (V + BB - 1) / BB;
+    // Bricks of BB x BB x depth sorted by the distance of their centre from
+    // the volume centre (ties by index): central bricks, which every
+    // direction's slab crosses, are dispatched first.
+    const int nb = (V + BB - 1) / BB, nz = (V + depth - 1) / depth;
     const double c = V / 2;
     struct Item { double d; int id; };
-    Item *items = new Item[(size_t)nb * nb * nb];
-    int n = 0;
-    for (int z = 0; z < nb; z++)
+    std::vector<Item> items;
+    items.reserve((size_t)nb * nb * nz);
+    for (int z = 0; z < nz; z++)
         for (int y = 0; y < nb; y++)
             for (int x = 0; x < nb; x++) {
                 const double dx = x * BB + 0.5 * (BB - 1) - c, dy = y * BB + 0.5 * (BB - 1) - c,
-                             dz = z * BB + 0.5 * (BB - 1) - c;
-                items[n] = {dx * dx + dy * dy + dz * dz, (z * nb + y) * nb + x};
-                n++;
+                             dz = z * depth + 0.5 * (depth - 1) - c;
+                items.push_back({dx * dx + dy * dy + dz * dz, (z * nb + y) * nb + x});
             }
-    std::sort(items, items + n, [](const Item &a, const Item &b) { return a.d < b.d || (a.d == b.d && a.id < b.id); });
-    for (int i = 0; i < n; i++) out[i] = items[i].id;
-    delete[] items;
+    std::sort(items.begin(), items.end(),
+              [](const Item &a, const Item &b) { return a.d < b.d || (a.d == b.d && a.id < b.id); });
+    for (size_t i = 0; i < items.size(); i++) out[i] = items[i].id;
+}
+
+static BPArgs bp_args(float *volAcc, float *densAcc, const ProjGeom &g, const float *axes, int nAxes, const float *casImgs)
+{
+    BPArgs a;
+    a.vol = volAcc; a.dens = densAcc; a.axes = axes; a.img = casImgs; a.ker = g.ker;
+    a.V = g.V; a.M = g.M; a.K = g.K; a.nAxes = nAxes;
+    a.maskR = ref_mask_radius(g.maskRadius); a.hw = g.kerHWidth;
+    proj_consts(g, a.kerScale, a.kerCenter, a.fW, a.convW);
+    a.maskD2 = mask_d2(a.maskR, g.V);
+    {
+        int r = 0;  // floor(sqrt(maskD2))
+        while ((long long)(r + 1) * (r + 1) <= (long long)a.maskD2) r++;
+        a.maskLo = a.maskD2 < 0 ? g.V : g.V / 2 - r;
+    }
+    // In-mask voxel: |v - c| <= maskR; orthonormal frame (to 1e-4): |u|, |v| <=
+    // 1.00005, and the FP32 evaluation of fi adds < 1e-3.  Then fi, fj >=
+    // M/2 - 1.00005 maskR - 1e-3, which must be >= 0.5 for floor(fi + 0.5) to be
+    // roundf(fi) (for 0.25 <= x < 0.5 an FP32 x + 0.5 can round up to 1).
+    a.posRound = ((double)(g.M / 2) - 1.00005 * (double)a.maskR - 1e-3 >= 0.5) ? 1 : 0;
+    // The column kernel's pixel lists and slab bounds allow 5e-3 of error in
+    // where the frame puts a voxel of the mask's radius.
+    a.orthTol = (float)std::min(1e-4, 2e-3 / std::max(1.0, (double)a.maskR));
+    a.check = nullptr;
+    a.order = nullptr;
+    a.perXcd = a.totalWork = 0;
+    return a;
 }
 
 hipError_t launch_back_project_adjoint(float *volAcc, const ProjGeom &g, const float *axes,
-                                       int nAxes, const float *casImgs, hipStream_t s, const unsigned *check)
+                                       int nAxes, const float *casImgs, hipStream_t s, const unsigned *check,
+                                       const unsigned *columns)
 {
     if (nAxes <= 0) return hipSuccess;
     FPArgs a;
     a.vol = nullptr; a.axes = axes; a.out = nullptr; a.ker = g.ker; a.check = nullptr;
+    a.columns = columns;
+    a.orthTol = bp_args(nullptr, nullptr, g, axes, nAxes, nullptr).orthTol;
     a.V = g.V; a.M = g.M; a.K = g.K; a.nAxes = nAxes;
     a.maskR = ref_mask_radius(g.maskRadius);
     proj_consts(g, a.kerScale, a.kerCenter, a.fW, a.convW);
@@ -2792,7 +3330,9 @@ hipError_t launch_back_project_adjoint(float *volAcc, const ProjGeom &g, const f
         if (work > 0xffffffffull / 2) return hipErrorInvalidValue;
         a.totalWork = (unsigned)work;
         a.perXcd = 0;
-        const dim3 grid((a.totalWork + 3) / 4), block(kThreads);
+        // one tile per wave; after the column launches usually nothing is left
+        const unsigned tiles = (a.totalWork + 3) / 4;
+        const dim3 grid(columns ? std::min(tiles, 8192u) : tiles), block(kThreads);
         if (fast) hipLaunchKernelGGL(adj_lds_kernel<true>, grid, block, 0, s, a, casImgs, volAcc);
         else hipLaunchKernelGGL(adj_lds_kernel<false>, grid, block, 0, s, a, casImgs, volAcc);
         return hipGetLastError();
@@ -2807,28 +3347,99 @@ hipError_t launch_back_project_adjoint(float *volAcc, const ProjGeom &g, const f
     return hipGetLastError();
 }
 
-hipError_t launch_back_project(float *volAcc, float *densAcc, const ProjGeom &g,
-                               const float *axes, int nAxes, const float *casImgs, hipStream_t s,
-                               const int *brickOrder, int orderLen)
+// Where the column kernels win (they cost more per block, bp_fast_kernel and
+// the tiles' atomics more per direction), ms by columns / by the other kernel,
+// random directions:
+//   back projection  N=64: 500 0.7/1.38 (100: 0.25/0.16); N=96: 256 0.66/0.76, 1,000 2.05/3.01;
+//     N=128: 256 1.10/0.89, 800 2.74/2.70, 1,500 4.80/5.13; N=192: 300 2.84/2.77, 600 4.77/5.21;
+//     N=256: 300 5.53/5.55
+//   transpose  N=64: 1,500 2.64/2.17; N=96: 256 0.93/0.81, 1,000 2.92/3.13; N=128: 256 1.48/1.60,
+//     800 3.77/5.00; N=192: 100 1.82/1.24, 600 6.33/7.33; N=256: 300 6.82/6.67
+bool uses_columns(const ProjGeom &g, int nAxes, ColKind kind)
+{
+    const bool adjoint = kind == ColKind::Adjoint;
+    const int least = adjoint ? (g.V < 190 ? INT_MAX : g.V < 230 ? 800 : g.V < 300 ? 256 : 500)
+                              : (g.V < 230 ? 256 : g.V < 300 ? 1000 : 500);
+    if (nAxes < least || !bp_uses_fast_path(g)) return false;
+    const BPArgs a = bp_args(nullptr, nullptr, g, nullptr, nAxes, nullptr);
+    if (a.maskD2 < 0) return false;
+    // The transpose's windows stay inside the volume (no wrap of the linear
+    // index) and its pixels inside the image.
+    if (adjoint)
+        return a.maskLo >= BP_FORM_A_MIN + 1 && (long long)a.maskD2 <= (long long)(g.M / 2 - 1) * (g.M / 2 - 1);
+    return a.posRound && a.maskLo >= BP_FORM_A_MIN;
+}
+
+// Waves per brick of bp_fast_kernel.  A small volume's bricks do not fill the
+// GPU, and the central ones, which every direction crosses, set the time:
+// eight waves halve it (N=64, 100 directions: 0.28 -> 0.16 ms; with the
+// density, 777: 2.26 -> 1.25 ms; N=96, 512: 1.53 -> 1.41 ms); elsewhere the
+// passes' leftover groups of more waves cost more (N=96, 64 directions: 0.19
+// -> 0.26 ms; N=128, 2,000: 6.9 -> 10.6 ms).
+static int bp_fast_waves(int V, int nAxes)
+{
+    return V <= 80 || (V <= 160 && nAxes >= 32) || (V <= 210 && nAxes >= 256) ? 8 : 4;
+}
+
+int col_depth(ColKind kind) { return bc_depth((int)kind); }
+
+hipError_t launch_check_back(const float *casImgs, const ProjGeom &g, const float *axes, int nAxes, bool planes,
+                             unsigned *check, hipStream_t s, const unsigned *finite)
+{
+    const BPArgs a = bp_args(nullptr, nullptr, g, axes, nAxes, casImgs);
+    const size_t n = finite ? 0 : (size_t)std::max(nAxes, 0) * g.M * g.M;
+    if (finite) hipLaunchKernelGGL(k_check_from, dim3(1), dim3(1), 0, s, finite, check);
+    else hipLaunchKernelGGL(k_check_table, dim3(1), dim3(kThreads), 0, s, g.ker, g.K, check, 3u);
+    if (nAxes <= 0) return hipGetLastError();
+    const unsigned grid = std::min(grid_for(std::max(n, (size_t)nAxes)), 4096u);
+    hipLaunchKernelGGL(k_check_back, dim3(grid), dim3(kThreads), 0, s, casImgs, n, axes, nAxes, a.orthTol, planes ? 1 : 0,
+                       check);
+    return hipGetLastError();
+}
+
+template <int MODE, int W>
+static void col_launches(const BPColArgs &a, unsigned blocks, hipStream_t s)
+{
+    hipLaunchKernelGGL((col_kernel<2, MODE, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+    hipLaunchKernelGGL((col_kernel<1, MODE, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+    hipLaunchKernelGGL((col_kernel<0, MODE, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+}
+
+hipError_t launch_columns(ColKind kind, float *volAcc, const ProjGeom &g, const float *axes, int nAxes,
+                          const float *casImgs, hipStream_t s, const int *order, int orderLen, const unsigned *check)
 {
     if (nAxes <= 0) return hipSuccess;
-    BPArgs a;
-    a.vol = volAcc; a.dens = densAcc; a.axes = axes; a.img = casImgs; a.ker = g.ker;
-    a.V = g.V; a.M = g.M; a.K = g.K; a.nAxes = nAxes;
-    a.maskR = ref_mask_radius(g.maskRadius); a.hw = g.kerHWidth;
-    proj_consts(g, a.kerScale, a.kerCenter, a.fW, a.convW);
-    const bool fast = bp_uses_fast_path(g);
-    a.maskD2 = mask_d2(a.maskR, g.V);
-    {
-        int r = 0;  // floor(sqrt(maskD2))
-        while ((long long)(r + 1) * (r + 1) <= (long long)a.maskD2) r++;
-        a.maskLo = a.maskD2 < 0 ? g.V : g.V / 2 - r;
+    if (!uses_columns(g, nAxes, kind) || !check || !order ||
+        orderLen != bp_brick_count(g.V, col_depth(kind)))
+        return hipErrorInvalidValue;
+    BPColArgs a;
+    a.b = bp_args(volAcc, nullptr, g, axes, nAxes, casImgs);
+    a.b.check = check;
+    a.b.order = order;
+    a.blocks8 = (g.V + BCN - 1) / BCN;
+    a.reachD2 = a.b.maskD2;
+    if (kind == ColKind::Adjoint) {
+        // pixels are within sqrt(maskD2) (times the frame's tolerance) of the
+        // centre, their voxels less than 2 further along each axis
+        const double r = std::sqrt((double)std::max(a.b.maskD2, 0)) * (1.0 + 1e-4) + 3.5;
+        a.reachD2 = (int)std::ceil(r * r);
     }
-    // In-mask voxel: |v - c| <= maskR; orthonormal frame (to 1e-4): |u|, |v| <=
-    // 1.00005, and the FP32 evaluation of fi adds < 1e-3.  Then fi, fj >=
-    // M/2 - 1.00005 maskR - 1e-3, which must be >= 0.5 for floor(fi + 0.5) to be
-    // roundf(fi) (for 0.25 <= x < 0.5 an FP32 x + 0.5 can round up to 1).
-    a.posRound = ((double)(g.M / 2) - 1.00005 * (double)a.maskR - 1e-3 >= 0.5) ? 1 : 0;
+    // Small volumes have few blocks, and the central ones' chain of directions
+    // sets the time: eight waves share it (N=64, 777 directions: 1.41 -> 1.00
+    // ms; N=96: 1.14 -> 1.31, N=128: 6.46 -> 6.80 for 2,000).
+    if (kind == ColKind::Adjoint) col_launches<COL_ADJOINT, 4>(a, (unsigned)orderLen, s);
+    else if (g.V <= 160) col_launches<COL_BACK, 8>(a, (unsigned)orderLen, s);
+    else col_launches<COL_BACK, 4>(a, (unsigned)orderLen, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_back_project(float *volAcc, float *densAcc, const ProjGeom &g,
+                               const float *axes, int nAxes, const float *casImgs, hipStream_t s,
+                               const int *brickOrder, int orderLen, const unsigned *check)
+{
+    if (nAxes <= 0) return hipSuccess;
+    BPArgs a = bp_args(volAcc, densAcc, g, axes, nAxes, casImgs);
+    const bool fast = bp_uses_fast_path(g);
     const int ex = fast ? BB : BPX, ey = fast ? BB : BPY, ez = fast ? BB : BPZ;
     a.bricksX = (g.V + ex - 1) / ex;
     const int bricksY = (g.V + ey - 1) / ey;
@@ -2837,13 +3448,18 @@ hipError_t launch_back_project(float *volAcc, float *densAcc, const ProjGeom &g,
     a.totalWork = (unsigned)a.bricksXY * (unsigned)bricksZ;
     a.perXcd = (a.totalWork + 7) / 8;
     a.order = brickOrder;
+    a.check = check;
     const dim3 grid(a.perXcd * 8), block(kThreads);
     if (fast) {
         if (!brickOrder || orderLen != (int)a.totalWork) return hipErrorInvalidValue;
         const dim3 g1(a.totalWork);
-        if (densAcc) hipLaunchKernelGGL(bp_fast_kernel<true>, g1, block, 0, s, a);
-        else hipLaunchKernelGGL(bp_fast_kernel<false>, g1, block, 0, s, a);
+        if (bp_fast_waves(g.V, nAxes) == 8) {
+            if (densAcc) hipLaunchKernelGGL((bp_fast_kernel<true, 8>), g1, dim3(512), 0, s, a);
+            else hipLaunchKernelGGL((bp_fast_kernel<false, 8>), g1, dim3(512), 0, s, a);
+        } else if (densAcc) hipLaunchKernelGGL((bp_fast_kernel<true, 4>), g1, block, 0, s, a);
+        else hipLaunchKernelGGL((bp_fast_kernel<false, 4>), g1, block, 0, s, a);
     } else {
+        if (check) return hipErrorInvalidValue;
         if (densAcc) hipLaunchKernelGGL(bp_kernel<true>, grid, block, 0, s, a);
         else hipLaunchKernelGGL(bp_kernel<false>, grid, block, 0, s, a);
     }
@@ -3011,7 +3627,7 @@ hipError_t launch_convert_volume(void *dst, int dtype, const float *src, size_t 
 hipError_t launch_check_volume(const void *vol, int dtype, size_t n, const float *ker, int K, unsigned *check,
                                hipStream_t s)
 {
-    hipLaunchKernelGGL(k_check_table, dim3(1), dim3(kThreads), 0, s, ker, K, check);
+    hipLaunchKernelGGL(k_check_table, dim3(1), dim3(kThreads), 0, s, ker, K, check, 1u);
     if (n == 0) return hipGetLastError();
     const dim3 grid(std::min(grid_for(n), 4096u)), block(kThreads);
     switch (dtype) {

@@ -512,7 +512,9 @@ struct mgg_server {
                 check_launch(launch_herm2d_to_cas(dHerm, dCas + a0 * mm, M, gN, p.stream), "herm2d_to_cas");
             }
             if (r.imgMem != Mem::Device) HIP_TRY(hipEventRecord(p.handoff[k & 1], p.stream));  // buffer free
-            check_launch(back_project_launch(dAcc, nullptr, g, dAxes + (size_t)9 * c0, cnt, dCas, p.stream),
+            // the half spectra are free again: the launch's flag goes there
+            check_launch(back_project_launch(dAcc, nullptr, g, dAxes + (size_t)9 * c0, cnt, dCas, p.stream,
+                                             reinterpret_cast<unsigned *>(dHerm)),
                          "back_project");
         }
         chain_cas_to_volume(dAcc, M, v.pad, dVol, N, precomp_for(M), 1, dReal3, dHerm3, p.stream);

@@ -183,8 +183,10 @@ def back_project(cas_images: torch.Tensor, axes: torch.Tensor, v: int, mask_radi
     ker = kb_table(cas_images.device) if ker is None else ker
     _check(ker, "ker")
     mr = default_mask_radius(m) if mask_radius is None else float(mask_radius)
-    _lib.call("mgg_op_back_project", _ptr(out), _ptr(density) if density is not None else None, v,
-              _ptr(axes), p, _ptr(cas_images), m, mr, _ptr(ker), ker.numel(), float(hwidth), _stream())
+    scratch = torch.empty(1, device=out.device, dtype=torch.int32)
+    _lib.call("mgg_op_back_project_scratch", _ptr(out), _ptr(density) if density is not None else None, v,
+              _ptr(axes), p, _ptr(cas_images), m, mr, _ptr(ker), ker.numel(), float(hwidth), _ptr(scratch),
+              _stream())
     return out
 
 
@@ -240,13 +242,16 @@ def back_project_adjoint(cas_images: torch.Tensor, axes: torch.Tensor, v: int, m
                   _ptr(ker), ker.numel(), float(hwidth), _stream())
         return out
     if check is None or check is True:
-        check = check_images(cas_images[:p], ker)
+        check = None
     else:
         _need_numel(check, 1, "check")
         _same_device(("cas_images", cas_images), ("check", check))
         _check(check, "check", torch.int32)
-    _lib.call("mgg_op_back_project_adjoint_checked", _ptr(out), v, _ptr(axes), p, _ptr(cas_images), m, mr,
-              _ptr(ker), ker.numel(), float(hwidth), _ptr(check), _stream())
+    # without a flag the call looks for itself (check_images' conditions)
+    scratch = torch.empty(1, device=out.device, dtype=torch.int32)
+    _lib.call("mgg_op_back_project_adjoint_scratch", _ptr(out), v, _ptr(axes), p, _ptr(cas_images), m, mr,
+              _ptr(ker), ker.numel(), float(hwidth), _ptr(check) if check is not None else None, _ptr(scratch),
+              _stream())
     return out
 
 
