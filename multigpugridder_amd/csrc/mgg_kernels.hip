@@ -135,6 +135,39 @@ template <> struct VolLoad<DT_F16> {
 // unrolled with one unaligned vector load per x-row; other widths use the
 // generic loop.
 // ---------------------------------------------------------------------------
+// n / d for n < 2^31 by a multiplication (d and so the shift wave-uniform).
+struct FastDiv {
+    unsigned d, mul, shift;
+    void set(unsigned div)
+    {
+        d = div;
+        unsigned l = 0;
+        while ((1ull << l) < div) l++;
+        shift = l + 31;
+        mul = (unsigned)(((1ull << shift) + div - 1) / div);
+    }
+    __device__ __forceinline__ unsigned operator()(unsigned n) const
+    {
+        return (unsigned)(((unsigned long long)n * mul) >> shift);
+    }
+};
+
+// fp_lds_kernel's order of the 8x8 tiles.  A workgroup takes 2 x 2 tiles, the
+// hardware deals workgroups round-robin to the 8 XCDs, and each XCD walks
+// whole images (or, for few directions, whole bands of images) of its own, so
+// that neighbouring tiles, whose voxel boxes overlap, share that XCD's L2.
+// Walking the tiles row by row over all XCDs kept vertical neighbours on one
+// XCD only where a row of workgroups is a multiple of 8 (N=64, 128, 256):
+// 500 random directions 1,280 -> 828 us at N=160, 1,743 -> 1,205 at N=192,
+// 2,048 at N=96 1,568 -> 1,208, 2,000 at N=128 2,183 -> 2,068.
+struct FPWalk {
+    FastDiv unitTiles;  // workgroup tiles of a unit (a band of one image)
+    FastDiv cols;       // workgroup tiles across an image
+    FastDiv bands;      // units per image
+    unsigned rows, bandRows;  // workgroup tile rows of an image, of a band
+    unsigned units, perXcd;   // units in all; workgroup tiles of one XCD's list
+};
+
 struct FPArgs {
     const void *vol;
     const float *axes;
@@ -146,6 +179,7 @@ struct FPArgs {
     unsigned perXcd, totalWork;
     int maskD2;  // fp_lds_kernel: largest integer d2 with sqrtf((float)d2) <= maskR (-1: none)
     const unsigned *check;  // fp_lds_kernel with the 501-entry table: launch_check_volume's flag, or null
+    FPWalk walk;            // fp_lds_kernel: its order of the tiles
     const unsigned *columns;  // adj_lds_kernel: launch_check_back's flag when the column launches came first, or null
     float orthTol;            // with columns: frames they took are orthonormal to this
 };
@@ -265,14 +299,12 @@ __global__ __launch_bounds__(kThreads) void fp_kernel(FPArgs p)
 // accumulation rounding differs.
 // ---------------------------------------------------------------------------
 constexpr int FPT = 8;          // tile edge (pixels)
-// Per-wave staged box budget (floats).  Four boxes take 40,960 bytes of LDS,
-// a quarter of the CU's 160 KB, so four workgroups share a CU (the kernel's
-// 121 VGPRs allow four waves per SIMD, at most 128 do); 73% of the 8x8 tiles' boxes fit whole
-// on the grid and random workloads at N=128 (median 2,400 floats), the rest
-// are staged as two 8x4 halves.  Occupancy matters more than the halves'
-// extra work: three workgroups per CU with a 3,392-float budget (nearly every
-// box whole) ran 31% slower, and 2,304 floats (45% whole) 8% slower.
-constexpr int FPBOX = 2560;     // per-wave staged box budget (floats)
+// Per-wave staged box budget (floats).  Four boxes and the phase table take
+// 40,928 bytes of LDS, a quarter of the CU's 160 KB, so four workgroups share a
+// CU (the kernel's 125 VGPRs allow four waves per SIMD, at most 128 do); nearly
+// every 8x8 tile's box of the 4x4x4 windows fits whole, the rest are staged as
+// two 8x4 halves.  Five workgroups per CU with 1,920 floats ran 10% slower.
+constexpr int FPBOX = 2432;     // per-wave staged box budget (floats)
 constexpr int FPKER = 640;      // generic-table path: table floats kept in LDS
 
 __device__ __forceinline__ void wave_lds_sync_fp()
@@ -345,8 +377,8 @@ __device__ __forceinline__ void load4<VolLoad<DT_F16>>(const uint16_t *p, float 
 // [floor(min) - 2, ceil(max) + 2], about 40% fewer voxels to stage.
 template <int DT, bool FAST, bool W4, bool BIG>
 __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *__restrict__ sker,
-                                                 float *__restrict__ box, int a, int i0, int j0, int ln,
-                                                 bool active, bool pix, float *out)
+                                                 const f4 *__restrict__ phase, float *__restrict__ box, int a, int i0,
+                                                 int j0, int ln, bool active, bool pix, float *out)
 {
     using L = VolLoad<DT>;
     using T = typename L::T;
@@ -360,26 +392,61 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
     const float x = ref_sum2c(u0, fi, v0, fj, (float)cv);
     const float y = ref_sum2c(u1, fi, v1, fj, (float)cv);
     const float z = ref_sum2c(u2, fi, v2, fj, (float)cv);
-    const int X = (int)roundf(x), Y = (int)roundf(y), Z = (int)roundf(z);
-    // first tap of each axis' window
-    const int Xs = X - 2 + ((W4 && x >= (float)X) ? 1 : 0);
-    const int Ys = Y - 2 + ((W4 && y >= (float)Y) ? 1 : 0);
-    const int Zs = Z - 2 + ((W4 && z >= (float)Z) ? 1 : 0);
+    // centre and first tap of each axis' window
+    int X = 0, Y = 0, Z = 0, Xs, Ys, Zs;
+    if (W4) {
+        Xs = (int)floorf(x) - 1; Ys = (int)floorf(y) - 1; Zs = (int)floorf(z) - 1;
+    } else {
+        X = (int)roundf(x); Y = (int)roundf(y); Z = (int)roundf(z);
+        Xs = X - 2; Ys = Y - 2; Zs = Z - 2;
+    }
 
     const long long V3 = (long long)V * V * V;
     const T *vol = (const T *)p.vol;
 
     float wi[NW], wj[NW], wk[NW];
+    bool single = true;
+    if constexpr (W4) {
+        // The four entries of an axis' window lie 125 apart: one index, of the
+        // last tap, and one row (T[k], T[k + 125], T[k + 250], T[k + 375]) of
+        // the phase table.  The first taps' indices are that one's minus
+        // multiples of 125 unless its FP32 value is exactly a half-integer
+        // (see ColVisit's argument) or the position below 1, where tap - x may
+        // be rounded; then every lane looks its taps up one by one.  One row
+        // read (5 ns per wave and CU) replaces four table gathers through the
+        // texture path (10 ns each); with the four-dword rows below 2,196 ->
+        // 1,997 us per 2,000 directions at N=128.
+        if (phase != nullptr) {
+            const float sx = fmaf((float)(Xs + 3) - x, 125.0f, 250.0f);
+            const float sy = fmaf((float)(Ys + 3) - y, 125.0f, 250.0f);
+            const float sz = fmaf((float)(Zs + 3) - z, 125.0f, 250.0f);
+            const bool odd = __builtin_amdgcn_fractf(sx) == 0.5f || __builtin_amdgcn_fractf(sy) == 0.5f ||
+                             __builtin_amdgcn_fractf(sz) == 0.5f || !(fminf(x, fminf(y, z)) >= 1.0f);
+            single = __ballot(active && odd) != 0ull;
+            // (clamped: a non-finite coordinate stays inside the table)
+            const f4 qx = phase[min(max(cvt_rpi(sx) - 375, 0), 125)];
+            const f4 qy = phase[min(max(cvt_rpi(sy) - 375, 0), 125)];
+            const f4 qz = phase[min(max(cvt_rpi(sz) - 375, 0), 125)];
 #pragma unroll
-    for (int t = 0; t < NW; t++) {
-        if (FAST) {
-            wi[t] = kb_fast_fp(p.ker, (float)(Xs + t) - x);
-            wj[t] = kb_fast_fp(p.ker, (float)(Ys + t) - y);
-            wk[t] = kb_fast_fp(p.ker, (float)(Zs + t) - z);
-        } else {
-            wi[t] = sker[kb_index((float)(Xs + t) - x, p.fW, p.kerScale, p.kerCenter, p.K)];
-            wj[t] = sker[kb_index((float)(Ys + t) - y, p.fW, p.kerScale, p.kerCenter, p.K)];
-            wk[t] = sker[kb_index((float)(Zs + t) - z, p.fW, p.kerScale, p.kerCenter, p.K)];
+            for (int t = 0; t < NW; t++) {
+                wi[t] = qx[t];
+                wj[t] = qy[t];
+                wk[t] = qz[t];
+            }
+        }
+    }
+    if (single) {
+#pragma unroll
+        for (int t = 0; t < NW; t++) {
+            if (FAST) {
+                wi[t] = kb_fast_fp(p.ker, (float)(Xs + t) - x);
+                wj[t] = kb_fast_fp(p.ker, (float)(Ys + t) - y);
+                wk[t] = kb_fast_fp(p.ker, (float)(Zs + t) - z);
+            } else {
+                wi[t] = sker[kb_index((float)(Xs + t) - x, p.fW, p.kerScale, p.kerCenter, p.K)];
+                wj[t] = sker[kb_index((float)(Ys + t) - y, p.fW, p.kerScale, p.kerCenter, p.K)];
+                wk[t] = sker[kb_index((float)(Zs + t) - z, p.fW, p.kerScale, p.kerCenter, p.K)];
+            }
         }
     }
 
@@ -412,9 +479,9 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         if (!(Dx >= NW && Dy >= NW && Dz >= NW && Dx <= 64 && Dy <= 64 && Dz <= 64 &&
               (BIG ? 64LL * V * V : V3) * (long long)sizeof(T) < (1LL << 32)))
             return false;
-        // 16-byte segments per box row: enough that the 8-wide read of a window
-        // (below) stays inside the row's staged segments.
-        const int segs = (Dx + 8 - NW) >> 2;
+        // 16-byte segments per box row; for the 5-wide windows enough that the
+        // 8-wide read (below) stays inside the row's staged segments.
+        const int segs = W4 ? (Dx + 3) >> 2 : (Dx + 8 - NW) >> 2;
         // LDS pitches (floats), multiples of 4 (16-byte rows).  When the box
         // still fits, the row and plane pitches are padded to an odd number
         // of 16-byte units so that the rows and planes a tile's pixels read
@@ -447,11 +514,11 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         const long long linLo = (long long)bz0 * VV + (long long)by0 * V + bx0;
         const long long linHi = (long long)(bz0 + Dz - 1) * VV + (long long)(by0 + Dy - 1) * V + bx0 + 4 * segs - 1;
         const bool boxIn = linLo >= 0 && linHi < V3;
-        // Six planes per batch: all loads of a batch are in flight before the
-        // first LDS store waits on them (2, 4 and 6 planes: 19.9, 18.5 and
-        // 18.3 ms per 10,000 directions at N=128 with the 5-wide windows; 8
-        // needs more than 128 VGPRs, three waves per SIMD instead of four,
-        // 22.0 ms).  The checked and unchecked variants are separate loops
+        // Four planes per batch (three with the 16-bit types' conversions): all
+        // loads of a batch are in flight before the first LDS store waits on
+        // them (2, 3, 4, 5 and 6 planes: 2.17, 2.10, 2.07, 2.08 and 2.08 ms per
+        // 2,000 directions at N=128; BF16, 500 at N=256: 2.49, 2.28, -, 2.45
+        // and 2.48 ms; 8 needs more than 128 VGPRs, three waves per SIMD).  The checked and unchecked variants are separate loops
         // (boxIn is wave-uniform).  The unchecked one addresses the volume by
         // a 32-bit byte offset from the volume's base, or (BIG: volumes of
         // 4 GB and more) from the box's first element; the checked one, which
@@ -459,7 +526,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // int linear index, or (BIG) a 64-bit one.
         const T *volBox = vol + ((BIG && boxIn) ? linLo : 0);
         using Lin = std::conditional_t<BIG, long long, int>;
-        constexpr int SB = 6;
+        constexpr int SB = DT == DT_F32 ? 4 : 3;
         const int lStep = G * VV, dStep = G * PP;
         for (int c = 0; c < nLanePass; c++) {
             const int q = ln + 64 * c;
@@ -508,7 +575,22 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
                 stage(std::false_type{});
             }
         }
-        // 16-byte gather: each NW-tap row is read as the two aligned 16-byte
+        // 4-wide windows: a row is four dwords (two paired reads, no
+        // alignment), 64 products instead of the 128 of aligned 16-byte units.
+        auto planeSum4 = [&](const float *bq, const float (&wx)[NW], const float (&wy)[NW], int cc) {
+            float sc = 0.f;
+#pragma unroll
+            for (int bb = 0; bb < NW; bb++) {
+                float v[4];
+                __builtin_memcpy(v, bq + cc * PP + bb * RP, 16);
+                float row = wx[0] * v[0];
+#pragma unroll
+                for (int aa = 1; aa < 4; aa++) row = fmaf(wx[aa], v[aa], row);
+                sc = fmaf(wy[bb], row, sc);
+            }
+            return sc;
+        };
+        // 5-wide windows: each 5-tap row is read as the two aligned 16-byte
         // units that contain it, [xo - o, xo - o + 8) with o = xo & 3, and the
         // x weights are shifted by o with zeros in the unused slots.  Since
         // xo <= Dx - NW, xo - o + 8 <= 4 * floor((Dx - NW) / 4) + 8, which
@@ -559,12 +641,17 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         bool gathered = false;
         if constexpr (!decltype(splitT)::value) {
             if (active && mine) {
-                const int xo = Xs - bx0, o = xo & 3;
+                const int xo = Xs - bx0, o = W4 ? 0 : xo & 3;
                 const float *bq = box + (Zs - bz0) * PP + (Ys - by0) * RP + (xo - o);
-                float w8[8][NW];
-                shifted(wi, wj, o, w8);
+                if constexpr (W4) {
 #pragma unroll
-                for (int cc = 0; cc < NW; cc++) res = fmaf(wk[cc], planeSum(bq, w8, cc), res);
+                    for (int cc = 0; cc < NW; cc++) res = fmaf(wk[cc], planeSum4(bq, wi, wj, cc), res);
+                } else {
+                    float w8[8][NW];
+                    shifted(wi, wj, o, w8);
+#pragma unroll
+                    for (int cc = 0; cc < NW; cc++) res = fmaf(wk[cc], planeSum(bq, w8, cc), res);
+                }
                 gathered = true;
             }
         } else {
@@ -588,13 +675,18 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
             const float k0 = mine ? wk[0] : pkA, k1 = mine ? wk[1] : pkB;
             float part = 0.f;
             if (mine ? active : pAct != 0) {
-                const int xo = gX - bx0, o = xo & 3;
+                const int xo = gX - bx0, o = W4 ? 0 : xo & 3;
                 const float *bq = box + (gZ - bz0) * PP + (gY - by0) * RP + (xo - o);
-                float w8[8][NW];
-                shifted(gwi, gwj, o, w8);
-                part = fmaf(k0, planeSum(bq, w8, 0), part);
-                part = fmaf(k1, planeSum(bq, w8, 1), part);
-                if (!W4 && mine) part = fmaf(wk[2], planeSum(bq, w8, 2), part);
+                if constexpr (W4) {
+                    part = fmaf(k0, planeSum4(bq, gwi, gwj, 0), part);
+                    part = fmaf(k1, planeSum4(bq, gwi, gwj, 1), part);
+                } else {
+                    float w8[8][NW];
+                    shifted(gwi, gwj, o, w8);
+                    part = fmaf(k0, planeSum(bq, w8, 0), part);
+                    part = fmaf(k1, planeSum(bq, w8, 1), part);
+                    if (mine) part = fmaf(wk[2], planeSum(bq, w8, 2), part);
+                }
             }
             const float other = __shfl_xor(part, 32);
             res = part + other;
@@ -652,12 +744,10 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
 // One 8x8 tile of one direction; W4 (only with the 501-entry table) selects
 // the 4-wide windows.
 template <int DT, bool FAST, bool W4, bool BIG = false>
-__device__ __forceinline__ void fp_lds_tile(const FPArgs &p, const float *__restrict__ sker, float *__restrict__ box,
-                                            unsigned work, int ln)
+__device__ __forceinline__ void fp_lds_tile(const FPArgs &p, const float *__restrict__ sker,
+                                            const f4 *__restrict__ phase, float *__restrict__ box, int a, int tx, int ty,
+                                            int ln)
 {
-    const int a = (int)(work / (unsigned)p.tilesPerImg);
-    const int tile = (int)(work - (unsigned)a * (unsigned)p.tilesPerImg);
-    const int ty = tile / p.tilesPerRow, tx = tile - ty * p.tilesPerRow;
     const int i0 = tx * FPT, j0 = ty * FPT;
     const int i = i0 + (ln & 7), j = j0 + (ln >> 3);
     const int M = p.M, ci = M / 2;
@@ -671,7 +761,7 @@ __device__ __forceinline__ void fp_lds_tile(const FPArgs &p, const float *__rest
         if (pix) *out = 0.f;
         return;
     }
-    fp_lds_tile_body<DT, FAST, FAST && W4, BIG>(p, sker, box, a, i0, j0, ln, active, pix, out);
+    fp_lds_tile_body<DT, FAST, FAST && W4, BIG>(p, sker, phase, box, a, i0, j0, ln, active, pix, out);
 }
 
 // The 4-wide windows need a finite volume and a finite 501-entry table whose
@@ -682,27 +772,51 @@ __device__ __forceinline__ bool fp_win4(const unsigned *check)
     return check != nullptr && __builtin_amdgcn_readfirstlane(*check) == 1u;
 }
 
+// Rows (T[k], T[k + 125], T[k + 250], T[k + 375]), k <= 125, of the 501-entry
+// table, by the whole workgroup.
+constexpr int FPPHASE = 126;
+__device__ __forceinline__ void fp_phase_table(f4 *__restrict__ phase, const float *__restrict__ ker)
+{
+    for (int k = threadIdx.x; k < FPPHASE; k += kThreads) {
+        const f4 row = {ker[k], ker[k + 125], ker[k + 250], ker[k + 375]};
+        phase[k] = row;
+    }
+    __syncthreads();
+}
+
 template <int DT, bool FAST, bool BIG>
 __global__ __launch_bounds__(kThreads) void fp_lds_kernel(FPArgs p)
 {
     __shared__ float sker[FPKER];
     __shared__ __attribute__((aligned(16))) float sbox[4][FPBOX];
+    __shared__ f4 sphase[FAST ? FPPHASE : 1];
 
     if (!FAST) {  // the fast lookup reads the table from global memory
         for (int t = threadIdx.x; t < p.K; t += kThreads) sker[t] = p.ker[t];
         __syncthreads();
     }
-    // Each wave takes work items wv + 4*blockIdx.x, + 4*gridDim.x, ...  (wave
-    // uniform, so the work index and its divisions stay scalar)
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+    const FPWalk &wk = p.walk;
+    const unsigned xcd = blockIdx.x & 7u;
+    auto walk = [&](auto win4) {
+        for (unsigned it = blockIdx.x >> 3; it < wk.perXcd; it += gridDim.x >> 3) {
+            const unsigned k = wk.unitTiles(it), t = it - k * wk.unitTiles.d;
+            const unsigned unit = xcd + 8u * k;
+            const unsigned a = wk.bands(unit), band = unit - a * wk.bands.d;
+            const unsigned r = wk.cols(t), row = band * wk.bandRows + r, col = t - r * wk.cols.d;
+            const int tx = (int)(2u * col) + (wv & 1), ty = (int)(2u * row) + (wv >> 1);
+            if (unit >= wk.units || row >= wk.rows || tx >= p.tilesPerRow || ty >= p.tilesPerRow) continue;
+            fp_lds_tile<DT, FAST, decltype(win4)::value, BIG>(p, sker, decltype(win4)::value ? sphase : nullptr, sbox[wv],
+                                                              (int)a, tx, ty, ln);
+        }
+    };
     // The window width is chosen once, outside the tile loop, so that each
     // loop is register-allocated on its own.
     if (FAST && fp_win4(p.check)) {
-        for (unsigned work = blockIdx.x * 4u + (unsigned)wv; work < p.totalWork; work += gridDim.x * 4u)
-            fp_lds_tile<DT, FAST, true, BIG>(p, sker, sbox[wv], work, ln);
+        fp_phase_table(sphase, p.ker);
+        walk(std::true_type{});
     } else {
-        for (unsigned work = blockIdx.x * 4u + (unsigned)wv; work < p.totalWork; work += gridDim.x * 4u)
-            fp_lds_tile<DT, FAST, false, BIG>(p, sker, sbox[wv], work, ln);
+        walk(std::false_type{});
     }
 }
 
@@ -769,7 +883,9 @@ template <int DT, bool BIG>
 __global__ __launch_bounds__(kThreads) void fp_lds_multi_kernel(FPMultiArgs m)
 {
     __shared__ __attribute__((aligned(16))) float sbox[4][FPBOX];
+    __shared__ f4 sphase[FPPHASE];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+    fp_phase_table(sphase, m.seg[0].ker);  // segments with another table look up tap by tap
     for (unsigned work = blockIdx.x * 4u + (unsigned)wv; work < m.totalWork; work += gridDim.x * 4u) {
         int lo = 0, hi = m.nSegs - 1;
         while (lo < hi) {
@@ -784,8 +900,12 @@ __global__ __launch_bounds__(kThreads) void fp_lds_multi_kernel(FPMultiArgs m)
         a.convW = 2; a.tilesPerRow = sg.tilesPerRow; a.tilesPerImg = sg.tilesPerImg;
         a.perXcd = 0; a.totalWork = 0; a.maskD2 = sg.maskD2; a.check = sg.check;
         a.columns = nullptr; a.orthTol = 0.f;
-        if (fp_win4(sg.check)) fp_lds_tile<DT, true, true, BIG>(a, nullptr, sbox[wv], work - sg.workStart, ln);
-        else fp_lds_tile<DT, true, false, BIG>(a, nullptr, sbox[wv], work - sg.workStart, ln);
+        const f4 *phase = sg.ker == m.seg[0].ker ? sphase : nullptr;
+        const unsigned local = work - sg.workStart;
+        const int d = (int)(local / (unsigned)sg.tilesPerImg), tile = (int)(local - (unsigned)d * (unsigned)sg.tilesPerImg);
+        const int ty = tile / sg.tilesPerRow, tx = tile - ty * sg.tilesPerRow;
+        if (fp_win4(sg.check)) fp_lds_tile<DT, true, true, BIG>(a, nullptr, phase, sbox[wv], d, tx, ty, ln);
+        else fp_lds_tile<DT, true, false, BIG>(a, nullptr, nullptr, sbox[wv], d, tx, ty, ln);
     }
 }
 
@@ -3160,11 +3280,24 @@ hipError_t launch_forward_project(const void *vol, int dtype, const ProjGeom &g,
         if (work > 0xffffffffull / 2) return hipErrorInvalidValue;
         a.totalWork = (unsigned)work;
         a.perXcd = 0;
-        // Three tiles per wave, a grid-stride apart (one workgroup per twelve
-        // tiles): 10.8 ms per 10,000 directions at N=128 against 12.1 ms with
-        // one tile per wave, 11.4 / 11.9 / 11.3 / 11.6 ms with 2 / 4 / 6 / 8
-        // tiles per wave, 13.5 ms with a persistent 1,024-workgroup grid.
-        const dim3 grid((a.totalWork + 11) / 12), block(kThreads);
+        // Units of whole images from 64 directions on; bands below, so that every
+        // XCD has work.
+        FPWalk &wk = a.walk;
+        const unsigned cols = (unsigned)(a.tilesPerRow + 1) / 2;
+        unsigned bands = 1;
+        while (bands < 8 && bands < cols && (unsigned)nAxes * bands < 64u) bands *= 2;
+        wk.rows = cols;
+        wk.bandRows = (cols + bands - 1) / bands;
+        wk.cols.set(cols);
+        wk.bands.set(bands);
+        wk.unitTiles.set(cols * wk.bandRows);
+        wk.units = (unsigned)nAxes * bands;
+        wk.perXcd = (wk.units + 7) / 8 * cols * wk.bandRows;
+        // Four tiles per wave, a stride of the grid apart: 2,000 random
+        // directions at N=128 in 2.32 / 2.12 / 2.06 / 2.07 / 2.09 ms with 1 /
+        // 2 / 3 / 4 / 6, 16 in 27 / 27 / 35 / 27 / 30 us.
+        const unsigned tpw = 4;
+        const dim3 grid((wk.perXcd + tpw - 1) / tpw * 8), block(kThreads);
         // volumes of 4 GB and more: box addressing from the box's first element
         const int esz = dtype == DT_F32 ? 4 : 2;
         const bool big = (long long)g.V * g.V * g.V * esz >= (1LL << 32);
