@@ -417,6 +417,12 @@ void chain_images_to_cas(const float *images, float *casImgs, float2 *herm, int 
 void chain_volume_to_cas(const float *vol, int nn, float *casVol, int m, int pad,
                          const float *dPrecomp, float *real3, float2 *herm3, hipStream_t s)
 {
+    if (fused_volume_supported(m, nn)) {
+        check_launch(launch_fused_volume_to_cas(vol, nn, casVol, m, pad, dPrecomp, herm3,
+                                                reinterpret_cast<float2 *>(real3), s),
+                     "fused_volume_to_cas");
+        return;
+    }
     check_launch(launch_vol_to_real3d(vol, nn, real3, m, dPrecomp, s), "vol_to_real3d");
     fft_exec(2, m, 1, real3, herm3, s);
     check_launch(launch_herm3d_to_casvol(herm3, m, casVol, m + 2 * pad, pad, s), "herm3d_to_casvol");
@@ -426,10 +432,16 @@ void chain_cas_to_volume(const float *casVol, int m, int pad, float *vol, int nn
                          const float *dPrecomp, int zeroNyq, float *real3, float2 *herm3,
                          hipStream_t s, bool transpose)
 {
+    const double scale = transpose ? 1.0 : 1.0 / ((double)m * (double)m * (double)m);
+    if (fused_volume_supported(m, nn)) {
+        check_launch(launch_fused_cas_to_volume(casVol, m, pad, vol, nn, dPrecomp, zeroNyq, (float)scale, herm3,
+                                                reinterpret_cast<float2 *>(real3), s),
+                     "fused_cas_to_volume");
+        return;
+    }
     check_launch(launch_casvol_to_herm3d(casVol, m + 2 * pad, pad, herm3, m, zeroNyq, s),
                  "casvol_to_herm3d");
     fft_exec(3, m, 1, herm3, real3, s);
-    const double scale = transpose ? 1.0 : 1.0 / ((double)m * (double)m * (double)m);
     check_launch(launch_real3d_to_vol(real3, m, vol, nn, dPrecomp, (float)scale, s), "real3d_to_vol");
 }
 

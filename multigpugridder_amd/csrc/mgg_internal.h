@@ -144,6 +144,14 @@ hipError_t launch_casvol_to_herm3d(const float *casVol, int V, int pad, float2 *
 hipError_t launch_real3d_to_vol(const float *real, int M, float *vol, int N,
                                 const float *precomp, float scale, hipStream_t s);
 
+// Fused volume chains (the image chains' M): a holds N * N * (M/2 + 1) float2,
+// b N * M * (M/2 + 1).
+bool fused_volume_supported(int M, int N);
+hipError_t launch_fused_volume_to_cas(const float *vol, int N, float *casVol, int M, int pad, const float *precomp,
+                                      float2 *a, float2 *b, hipStream_t s);
+hipError_t launch_fused_cas_to_volume(const float *casVol, int M, int pad, float *vol, int N, const float *precomp,
+                                      int zeroNyquist, float scale, float2 *a, float2 *b, hipStream_t s);
+
 // ---- reductions, conversions, fills --------------------------------------
 // out[i] = sum_p parts[p*stride + i] accumulated in FP64 (partial volumes).
 hipError_t launch_reduce_partials(float *out, const float *parts, int nParts, size_t n,

@@ -2916,6 +2916,256 @@ __global__ void k_real3d_to_vol(const float *__restrict__ real, int M, float *__
 }
 
 // ---------------------------------------------------------------------------
+// Fused volume chains for the image chains' sizes (M = 128, 192, 256, 384 and
+// 512): three passes of one-dimensional transforms (fft_m) that neither read
+// nor write the padding.  With A = N x N x H and B = N x M x H complex values
+// (H = M/2 + 1, kx fastest) the forward chain goes volume -> A (along x, two
+// real rows in one complex transform) -> B (along y) -> CAS volume (along z,
+// each value written with its Hermitian mirror), the inverse back the same
+// way, keeping N of M outputs along z, y and x.  rocFFT's chain makes seven
+// passes over M^3 or V^3 values instead.  Along y and z a workgroup takes 16
+// neighbouring kx (lanes: kx fastest, so every load and store is a run of 16),
+// and workgroups of one (y, z) line of tiles follow each other on one XCD, so
+// that partial lines meet in its L2.  Bound by memory: along z at N=256 3.4 TB/s
+// (241 us forward, 825 MB) and 3.1 TB/s (inverse) of the 5.1 TB/s of a copy.
+// Both directions together: N=128 437 -> 111 us, N=256 3,835 -> 806 us.
+// ---------------------------------------------------------------------------
+struct VolLine { int line, kx0; bool ok; };
+// The workgroup's line (of n) and its first kx; n * tiles workgroups, rounded
+// up to 8 lines.
+template <int H>
+__device__ __forceinline__ VolLine vol_line(int n)
+{
+    constexpr int T = (H + 15) / 16;
+    const int idx = (int)(blockIdx.x >> 3), q = idx / T;
+    const int line = q * 8 + (int)(blockIdx.x & 7u);
+    return {line, 16 * (idx - q * T), line < n};
+}
+
+// Volume -> A.  Grid: 32 rows per workgroup.
+template <int R>
+__global__ __launch_bounds__(256) void k_vol_fwd_x(const float *__restrict__ vol, int N, float2 *__restrict__ A,
+                                                   const float *__restrict__ pc)
+{
+    using G = FftGeom<R>;
+    constexpr int M = G::M, H = G::H;
+    __shared__ float2 sx[16 * G::FFB];
+    __shared__ float2 tw[M];
+    load_tw<R>(tw);
+    const int tid = threadIdx.x, f = tid >> 4, t = tid & 15;
+    const int off = (M - N) / 2, rows = N * N;
+    const int row0 = 32 * (int)blockIdx.x + 2 * f;
+    float2 *ex = sx + f * G::FFB;
+    float2 v[R];
+    {
+        const int r0 = min(row0, rows - 1), r1 = min(row0 + 1, rows - 1);
+        const int z0 = r0 / N + off, y0 = r0 % N + off, z1 = r1 / N + off, y1 = r1 % N + off;
+        const double w0 = (double)pc[y0] * (double)pc[z0], w1 = (double)pc[y1] * (double)pc[z1];
+        const float s0 = chk(y0 + z0), s1 = chk(y1 + z1);
+        float a[R], b[R];
+#pragma unroll
+        for (int n2 = 0; n2 < R; n2++) {  // unconditional loads from clamped addresses
+            const int q = min(max(t + 16 * n2 - off, 0), N - 1);
+            a[n2] = vol[(size_t)r0 * N + q];
+            b[n2] = vol[(size_t)r1 * N + q];
+        }
+#pragma unroll
+        for (int n2 = 0; n2 < R; n2++) {
+            const int mx = t + 16 * n2, q = mx - off;
+            const bool in = q >= 0 && q < N;
+            const double px = (double)pc[mx];
+            const float sg = chk(mx);
+            v[n2] = make_float2(in ? sg * s0 * (float)(px * w0 * (double)a[n2]) : 0.f,
+                                in ? sg * s1 * (float)(px * w1 * (double)b[n2]) : 0.f);
+        }
+    }
+    __syncthreads();
+    fft_m<R, -1>(v, t, ex, tw);
+#pragma unroll
+    for (int m = 0; m < R; m++) ex[out_idx<R>(t, m)] = v[out_slot<R>(m)];
+    __syncthreads();
+    for (int r = tid >> 6; r < 32; r += 4) {
+        const int row = 32 * (int)blockIdx.x + r;
+        if (row >= rows) break;
+        const float2 *zf = sx + (r >> 1) * G::FFB;
+        for (int k = tid & 63; k < H; k += 64) {
+            const float2 z = zf[k], zm = zf[mirror_idx<M>(k)];
+            A[(size_t)row * H + k] = (r & 1) ? make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x))
+                                             : make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));
+        }
+    }
+}
+
+// A <-> B, lines z (S = -1: N values of y in, M out; S = 1: M in, N out).
+template <int R, int S>
+__global__ __launch_bounds__(256) void k_vol_y(const float2 *__restrict__ in, float2 *__restrict__ out, int N)
+{
+    using G = FftGeom<R>;
+    constexpr int M = G::M, H = G::H;
+    __shared__ float2 sx[16 * G::FFB];
+    __shared__ float2 tw[M];
+    load_tw<R>(tw);
+    const VolLine l = vol_line<H>(N);
+    if (!l.ok) return;  // uniform
+    const int tid = threadIdx.x, f = tid & 15, t = tid >> 4, kx = l.kx0 + f, off = (M - N) / 2;
+    const int nIn = S < 0 ? N : M, oIn = S < 0 ? off : 0, nOut = S < 0 ? M : N, oOut = S < 0 ? 0 : off;
+    const float2 *src = in + (size_t)l.line * nIn * H + min(kx, H - 1);
+    float2 v[R];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) v[n2] = src[(size_t)min(max(t + 16 * n2 - oIn, 0), nIn - 1) * H];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) {
+        const int y = t + 16 * n2 - oIn;
+        if (y < 0 || y >= nIn) v[n2] = make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    fft_m<R, S>(v, t, sx + f * G::FFB, tw);
+    if (kx < H) {
+        float2 *dst = out + (size_t)l.line * nOut * H + kx;
+#pragma unroll
+        for (int m = 0; m < R; m++) {
+            const int y = out_idx<R>(t, m) - oOut;
+            if (y >= 0 && y < nOut) dst[(size_t)y * H] = v[out_slot<R>(m)];
+        }
+    }
+}
+
+// B -> CAS volume, lines ky; the padding shell is k_casvol_shell's.
+template <int R>
+__global__ __launch_bounds__(256) void k_vol_fwd_z(const float2 *__restrict__ B, int N, float *__restrict__ casVol, int V,
+                                                   int pad, float gsign)
+{
+    using G = FftGeom<R>;
+    constexpr int M = G::M, H = G::H;
+    __shared__ float2 sx[16 * G::FFB];
+    __shared__ float2 tw[M];
+    load_tw<R>(tw);
+    const VolLine l = vol_line<H>(M);
+    if (!l.ok) return;  // uniform
+    const int tid = threadIdx.x, f = tid & 15, t = tid >> 4, kx = l.kx0 + f, ky = l.line, off = (M - N) / 2;
+    const float2 *src = B + (size_t)ky * H + min(kx, H - 1);
+    float2 v[R];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) v[n2] = src[(size_t)min(max(t + 16 * n2 - off, 0), N - 1) * M * H];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) {
+        const int z = t + 16 * n2 - off;
+        if (z < 0 || z >= N) v[n2] = make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    fft_m<R, -1>(v, t, sx + f * G::FFB, tw);
+    if (kx >= H) return;
+    const bool mirror = kx != 0 && kx != M / 2;
+    const int my = mirror_idx<M>(ky);
+#pragma unroll
+    for (int m = 0; m < R; m++) {
+        const int kz = out_idx<R>(t, m);
+        const float2 F = v[out_slot<R>(m)];
+        const float s = gsign * chk(kx + ky + kz);  // the mirror's indices have the same parity
+        casVol[((size_t)(kz + pad) * V + (ky + pad)) * V + (kx + pad)] = s * F.x + s * F.y;
+        if (mirror)
+            casVol[((size_t)(mirror_idx<M>(kz) + pad) * V + (my + pad)) * V + (M - kx + pad)] = s * F.x - s * F.y;
+    }
+}
+
+// The CAS volume's padding: rows outside the M x M centre whole, the others'
+// ends.  Grid (V planes, 8), a row per wave.
+__global__ __launch_bounds__(256) void k_casvol_shell(float *__restrict__ casVol, int V, int pad)
+{
+    const int z = (int)blockIdx.x, ln = threadIdx.x & 63;
+    for (int y = (int)blockIdx.y * 4 + (int)(threadIdx.x >> 6); y < V; y += (int)gridDim.y * 4) {
+        float *row = casVol + ((size_t)z * V + y) * V;
+        const bool inside = y >= pad && y < V - pad && z >= pad && z < V - pad;
+        for (int x = ln; x < (inside ? 2 * pad : V); x += 64) row[inside && x >= pad ? V - 2 * pad + x : x] = 0.f;
+    }
+}
+
+// CAS volume -> B, lines ky.
+template <int R>
+__global__ __launch_bounds__(256) void k_vol_inv_z(const float *__restrict__ casVol, int V, int pad,
+                                                   float2 *__restrict__ B, int N, int zeroNyq)
+{
+    using G = FftGeom<R>;
+    constexpr int M = G::M, H = G::H;
+    __shared__ float2 sx[16 * G::FFB];
+    __shared__ float2 tw[M];
+    load_tw<R>(tw);
+    const VolLine l = vol_line<H>(M);
+    if (!l.ok) return;  // uniform
+    const int tid = threadIdx.x, f = tid & 15, t = tid >> 4, kx = l.kx0 + f, ky = l.line, off = (M - N) / 2;
+    const int xs = min(kx, H - 1), my = mirror_idx<M>(ky), mx = mirror_idx<M>(xs);
+    const float *p1 = casVol + ((size_t)pad * V + (ky + pad)) * V + (xs + pad);
+    const float *p2 = casVol + ((size_t)pad * V + (my + pad)) * V + (mx + pad);
+    const size_t VV = (size_t)V * V;
+    float c1[R], c2[R];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) {
+        const int kz = t + 16 * n2;
+        c1[n2] = p1[kz * VV];
+        c2[n2] = p2[mirror_idx<M>(kz) * VV];
+    }
+    float2 v[R];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) {
+        const int kz = t + 16 * n2;
+        const float s = (zeroNyq && (kx == 0 || ky == 0 || kz == 0)) ? 0.f : chk(kx + ky + kz);
+        v[n2] = make_float2(s * (0.5f * (c1[n2] + c2[n2])), s * (0.5f * (c1[n2] - c2[n2])));
+    }
+    __syncthreads();
+    fft_m<R, 1>(v, t, sx + f * G::FFB, tw);
+    if (kx >= H) return;
+    float2 *dst = B + (size_t)ky * H + kx;
+#pragma unroll
+    for (int m = 0; m < R; m++) {
+        const int z = out_idx<R>(t, m) - off;
+        if (z >= 0 && z < N) dst[(size_t)z * M * H] = v[out_slot<R>(m)];
+    }
+}
+
+// A -> volume: two Hermitian rows per complex transform, whose real and
+// imaginary outputs are the two real rows.  Grid: 32 rows per workgroup.
+template <int R>
+__global__ __launch_bounds__(256) void k_vol_inv_x(const float2 *__restrict__ A, float *__restrict__ vol, int N,
+                                                   const float *__restrict__ pc, double scale)
+{
+    using G = FftGeom<R>;
+    constexpr int M = G::M, H = G::H;
+    __shared__ float2 sx[16 * G::FFB];
+    __shared__ float2 tw[M];
+    load_tw<R>(tw);
+    const int tid = threadIdx.x, f = tid >> 4, t = tid & 15;
+    const int off = (M - N) / 2, rows = N * N;
+    const int row0 = 32 * (int)blockIdx.x + 2 * f;
+    const int r0 = min(row0, rows - 1), r1 = min(row0 + 1, rows - 1);
+    const float2 *a0 = A + (size_t)r0 * H, *a1 = A + (size_t)r1 * H;
+    float2 v[R];
+#pragma unroll
+    for (int n2 = 0; n2 < R; n2++) {
+        const int k = t + 16 * n2;
+        const bool up = k > M / 2;
+        const float2 p = a0[up ? M - k : k], q = a1[up ? M - k : k];
+        v[n2] = up ? make_float2(p.x + q.y, q.x - p.y) : make_float2(p.x - q.y, p.y + q.x);
+        // a real transform has no imaginary part at k = 0 and M/2
+        if (k == 0 || k == M / 2) v[n2] = make_float2(p.x, q.x);
+    }
+    __syncthreads();
+    fft_m<R, 1>(v, t, sx + f * G::FFB, tw);
+    const int z0 = r0 / N + off, y0 = r0 % N + off, z1 = r1 / N + off, y1 = r1 % N + off;
+    const double w0 = (double)pc[y0] * (double)pc[z0] * scale, w1 = (double)pc[y1] * (double)pc[z1] * scale;
+    const float s0 = chk(y0 + z0), s1 = chk(y1 + z1);
+#pragma unroll
+    for (int m = 0; m < R; m++) {
+        const int mx = out_idx<R>(t, m), px = mx - off;
+        if (px < 0 || px >= N) continue;
+        const float2 z = v[out_slot<R>(m)];
+        const double w = (double)pc[mx];
+        const float sg = chk(mx);
+        if (row0 < rows) vol[(size_t)row0 * N + px] = sg * s0 * (float)(w * w0 * (double)z.x);
+        if (row0 + 1 < rows) vol[(size_t)(row0 + 1) * N + px] = sg * s1 * (float)(w * w1 * (double)z.y);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Reductions, conversions, fills.
 // ---------------------------------------------------------------------------
 __global__ void k_reduce_partials(float *__restrict__ out, const float *__restrict__ parts,
@@ -3686,6 +3936,67 @@ hipError_t launch_fused_images_to_cas(const float *imgs, float2 *tmp, float *cas
     case 256: fused_forward<16>(imgs, tmp, cas, N, n, scale, zeroNyq, s); break;
     case 384: fused_forward<24>(imgs, tmp, cas, N, n, scale, zeroNyq, s); break;
     default: fused_forward<32>(imgs, tmp, cas, N, n, scale, zeroNyq, s); break;
+    }
+    return hipGetLastError();
+}
+
+bool fused_volume_supported(int M, int N)
+{
+    // B (N M H complex) has to fit the M^3 real scratch
+    return fused_chain_supported(M, N) && N % 2 == 0 && (size_t)N * (M + 2) <= (size_t)M * M;
+}
+
+template <int R>
+static void fused_vol_fwd(const float *vol, int N, float *casVol, int V, int pad, const float *pc, float2 *A, float2 *B,
+                          float gsign, hipStream_t s)
+{
+    constexpr int M = 16 * R, T = (M / 2 + 1 + 15) / 16;
+    const unsigned rows = (unsigned)((N * N + 31) / 32);
+    hipLaunchKernelGGL(k_vol_fwd_x<R>, dim3(rows), dim3(256), 0, s, vol, N, A, pc);
+    hipLaunchKernelGGL((k_vol_y<R, -1>), dim3((unsigned)((N + 7) / 8 * 8 * T)), dim3(256), 0, s, A, B, N);
+    if (pad > 0)
+        hipLaunchKernelGGL(k_casvol_shell, dim3((unsigned)V, 8), dim3(256), 0, s, casVol, V, pad);
+    hipLaunchKernelGGL(k_vol_fwd_z<R>, dim3((unsigned)(M * T)), dim3(256), 0, s, B, N, casVol, V, pad, gsign);
+}
+
+template <int R>
+static void fused_vol_inv(const float *casVol, int V, int pad, float *vol, int N, const float *pc, float2 *A, float2 *B,
+                          int zeroNyq, double scale, hipStream_t s)
+{
+    constexpr int M = 16 * R, T = (M / 2 + 1 + 15) / 16;
+    hipLaunchKernelGGL(k_vol_inv_z<R>, dim3((unsigned)(M * T)), dim3(256), 0, s, casVol, V, pad, B, N, zeroNyq);
+    hipLaunchKernelGGL((k_vol_y<R, 1>), dim3((unsigned)((N + 7) / 8 * 8 * T)), dim3(256), 0, s, B, A, N);
+    hipLaunchKernelGGL(k_vol_inv_x<R>, dim3((unsigned)((N * N + 31) / 32)), dim3(256), 0, s, A, vol, N, pc, scale);
+}
+
+hipError_t launch_fused_volume_to_cas(const float *vol, int N, float *casVol, int M, int pad, const float *precomp,
+                                      float2 *a, float2 *b, hipStream_t s)
+{
+    if (!fused_volume_supported(M, N)) return hipErrorInvalidValue;
+    const float g = ((3 * (M / 2)) & 1) ? -1.f : 1.f;
+    const int V = M + 2 * pad;
+    switch (M) {
+    case 128: fused_vol_fwd<8>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
+    case 192: fused_vol_fwd<12>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
+    case 256: fused_vol_fwd<16>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
+    case 384: fused_vol_fwd<24>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
+    default: fused_vol_fwd<32>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_fused_cas_to_volume(const float *casVol, int M, int pad, float *vol, int N, const float *precomp,
+                                      int zeroNyquist, float scale, float2 *a, float2 *b, hipStream_t s)
+{
+    if (!fused_volume_supported(M, N)) return hipErrorInvalidValue;
+    const double sc = (((3 * (M / 2)) & 1) ? -1.0 : 1.0) * (double)scale;
+    const int V = M + 2 * pad;
+    switch (M) {
+    case 128: fused_vol_inv<8>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;
+    case 192: fused_vol_inv<12>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;
+    case 256: fused_vol_inv<16>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;
+    case 384: fused_vol_inv<24>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;
+    default: fused_vol_inv<32>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;
     }
     return hipGetLastError();
 }
