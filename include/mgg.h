@@ -222,7 +222,9 @@ int mgg_op_back_project_adjoint_scratch(float *cas_volume, int v, const float *a
                                         const float *ker, int ker_size, float ker_hwidth,
                                         const unsigned *check, unsigned *scratch, void *stream);
 /* Gridders/gpuGridder.cpp:432-518: n CAS images (m x m) -> images (nn x nn).
- * Uses a batched rocFFT C2R; cas_images is clobbered (used as scratch). */
+ * cas_images may be clobbered (used as scratch); it is only read where
+ * mgg_op_image_chain_reads_only(m, nn) is 1. */
+int mgg_op_image_chain_reads_only(int m, int nn);
 int mgg_op_cas_images_to_images(float *cas_images, float *images, int n, int m, int nn,
                                 void *stream);
 /* No counterpart in the reference.  For callers that cannot allocate device

@@ -99,6 +99,7 @@ _SIGS = {
     "mgg_op_back_project_adjoint_scratch": [_vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp, _vp, _vp],
     "mgg_op_back_project_adjoint_checked": [_vp, _ci, _vp, _ci, _vp, _ci, _cf, _vp, _ci, _cf, _vp, _vp],
     "mgg_op_check_images": [_vp, _ci, _ci, _vp, _ci, _vp, _vp],
+    "mgg_op_image_chain_reads_only": [_ci, _ci],
     "mgg_op_cas_images_to_images": [_vp, _vp, _ci, _ci, _ci, _vp],
     "mgg_op_cas_images_to_images_noalloc": [_vp, _vp, _ci, _ci, _ci, _vp],
     "mgg_op_images_to_cas_images": [_vp, _vp, _ci, _ci, _ci, _vp],
@@ -199,6 +200,11 @@ def check(status: int) -> None:
 def call(name: str, *args) -> None:
     """Call an int-returning entry point and raise MggError on failure."""
     check(getattr(lib(), name)(*args))
+
+
+def image_chain_reads_only(m: int, n: int) -> bool:
+    """Whether the inverse image chain of these sizes leaves its input as it is."""
+    return bool(lib().mgg_op_image_chain_reads_only(m, n))
 
 
 def device_count() -> int:

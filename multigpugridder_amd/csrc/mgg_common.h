@@ -134,6 +134,12 @@ hipError_t back_project_launch(float *vol, float *dens, const ProjGeom &g, const
 // check: as above.
 hipError_t back_project_adjoint_launch(float *vol, const ProjGeom &g, const float *axes, int n, const float *casImgs,
                                        hipStream_t s, const unsigned *finite, unsigned *check);
+// Images a chain call takes with half spectra of kFftBatch images as scratch:
+// the two-pass chains keep only nn of the m columns between their passes.
+inline int image_batch(int m, int nn)
+{
+    return image_chain_supported(m, nn) ? (int)(kFftBatch * (size_t)m / (size_t)nn) : (int)kFftBatch;
+}
 void chain_cas_to_images(float *casImgs, float2 *herm, float *images, int n, int m, int nn,
                          hipStream_t s);
 // scale / zeroNyq: see launch_herm2d_to_cas (1 / 0 for ImgsToCASImgs itself).

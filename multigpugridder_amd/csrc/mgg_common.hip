@@ -386,7 +386,7 @@ void chain_cas_to_images(float *casImgs, float2 *herm, float *images, int n, int
                          hipStream_t s)
 {
     if (n <= 0) return;
-    if (fused_chain_supported(m, nn)) {
+    if (image_chain_supported(m, nn)) {
         check_launch(launch_fused_cas_to_images(casImgs, herm, images, m, nn, n, 1.0f / ((float)m * (float)m), s),
                      "fused_cas_to_images");
         return;
@@ -403,7 +403,7 @@ void chain_images_to_cas(const float *images, float *casImgs, float2 *herm, int 
                          hipStream_t s, float scale, int zeroNyq)
 {
     if (n <= 0) return;
-    if (fused_chain_supported(m, nn)) {
+    if (image_chain_supported(m, nn)) {
         check_launch(launch_fused_images_to_cas(images, herm, casImgs, m, nn, n, scale, zeroNyq, s),
                      "fused_images_to_cas");
         return;

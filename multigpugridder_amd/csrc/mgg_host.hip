@@ -828,6 +828,8 @@ int mgg_op_check_images(const float *cas_images, int n_images, int m, const floa
 }
 
 
+int mgg_op_image_chain_reads_only(int m, int nn) { return image_chain_supported(m, nn) ? 1 : 0; }
+
 int mgg_op_cas_images_to_images(float *cas_images, float *images, int n, int m, int nn, void *stream)
 {
     return guarded([&] {
@@ -837,8 +839,9 @@ int mgg_op_cas_images_to_images(float *cas_images, float *images, int n, int m, 
             raise(MGG_ERR_INVALID_ARGUMENT, "bad sizes n=%d m=%d nn=%d", n, m, nn);
         hipStream_t s = as_stream(stream);
         float2 *herm = scratch_herm(sizeof(float2) * (size_t)std::min<size_t>(n, kFftBatch) * m * (m / 2 + 1), s);
-        for (int a = 0; a < n; a += (int)kFftBatch) {
-            const int b = std::min<int>((int)kFftBatch, n - a);
+        const int most = image_batch(m, nn);
+        for (int a = 0; a < n; a += most) {
+            const int b = std::min(most, n - a);
             chain_cas_to_images(cas_images + (size_t)a * m * m, herm, images + (size_t)a * nn * nn, b, m, nn, s);
         }
     });
@@ -922,8 +925,9 @@ int mgg_op_images_to_cas_images(const float *images, float *cas_images, int n, i
             raise(MGG_ERR_INVALID_ARGUMENT, "bad sizes n=%d m=%d nn=%d", n, m, nn);
         hipStream_t s = as_stream(stream);
         float2 *herm = scratch_herm(sizeof(float2) * (size_t)std::min<size_t>(n, kFftBatch) * m * (m / 2 + 1), s);
-        for (int a = 0; a < n; a += (int)kFftBatch) {
-            const int b = std::min<int>((int)kFftBatch, n - a);
+        const int most = image_batch(m, nn);
+        for (int a = 0; a < n; a += most) {
+            const int b = std::min(most, n - a);
             chain_images_to_cas(images + (size_t)a * nn * nn, cas_images + (size_t)a * m * m, herm, b, m, nn, s);
         }
     });
@@ -941,8 +945,9 @@ int mgg_op_cas_images_to_images_transpose(const float *images, float *cas_images
         hipStream_t s = as_stream(stream);
         float2 *herm = scratch_herm(sizeof(float2) * (size_t)std::min<size_t>(n, kFftBatch) * m * (m / 2 + 1), s);
         const float scale = (float)(1.0 / ((double)m * (double)m));
-        for (int a = 0; a < n; a += (int)kFftBatch) {
-            const int b = std::min<int>((int)kFftBatch, n - a);
+        const int most = image_batch(m, nn);
+        for (int a = 0; a < n; a += most) {
+            const int b = std::min(most, n - a);
             chain_images_to_cas(images + (size_t)a * nn * nn, cas_images + (size_t)a * m * m, herm, b, m, nn, s,
                                 scale, 1);
         }

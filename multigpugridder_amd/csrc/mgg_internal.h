@@ -122,7 +122,10 @@ hipError_t launch_imgs_to_real2d(const float *imgs, float *real, int M, int N, i
 // zeroNyq the index-0 row and column of every CAS image are written as 0.
 hipError_t launch_herm2d_to_cas(const float2 *herm, float *cas, int M, int n, hipStream_t s,
                                 float scale = 1.f, int zeroNyq = 0);
-// Fused two-pass image chains (M = 256): tmp holds n * N * (M/2 + 1) float2.
+// Two-pass image chains: tmp holds n * N * (M/2 + 1) float2.  image_chain_supported:
+// any even M up to 512 with prime factors up to 13; fused_chain_supported: those
+// with kernels of their own (M = 128, 192, 256, 384, 512).
+bool image_chain_supported(int M, int N);
 bool fused_chain_supported(int M, int N);
 hipError_t launch_fused_cas_to_images(const float *cas, float2 *tmp, float *imgs, int M, int N, int n,
                                       float scale, hipStream_t s);
@@ -144,7 +147,7 @@ hipError_t launch_casvol_to_herm3d(const float *casVol, int V, int pad, float2 *
 hipError_t launch_real3d_to_vol(const float *real, int M, float *vol, int N,
                                 const float *precomp, float scale, hipStream_t s);
 
-// Fused volume chains (the image chains' M): a holds N * N * (M/2 + 1) float2,
+// Fused volume chains (M as image_chain_supported): a holds N * N * (M/2 + 1) float2,
 // b N * M * (M/2 + 1).
 bool fused_volume_supported(int M, int N);
 hipError_t launch_fused_volume_to_cas(const float *vol, int N, float *casVol, int M, int pad, const float *precomp,

@@ -2823,6 +2823,289 @@ __global__ __launch_bounds__(256) void k_fwd_rows(const float2 *__restrict__ tmp
 }
 
 // ---------------------------------------------------------------------------
+// The same two-pass image chains (and the volume chains below) for any other
+// even M up to 512 whose prime factors are 2, 3, 5, 7, 11 and 13: the
+// transforms run in place in LDS as Stockham passes of radix 10, 8, 6, 4, 2,
+// 3, 5, 7, 11 or 13.  A pass reads its butterflies into registers,
+// synchronises and writes them back in order.  rocFFT's chain costs five or
+// six passes over the padded images and, per call, up to 9 batch sizes of two
+// launches each.  300 images, there and back, from rocFFT's chain: M = 50
+// 93 -> 21 us, 100 154 -> 39, 200 284 -> 90, 300 695 -> 171, 480 1,674 -> 392
+// (3.4 TB/s of the bytes); one image 22-45 -> 17-25 us, launches on both sides.
+// A volume, there and back: M = 100 72 -> 40 us, 240 354 -> 127, 300 749 -> 212.
+// ---------------------------------------------------------------------------
+struct GPass {
+    FastDiv ns, count;   // product of the radices before; butterflies of a transform (M / radix)
+    unsigned radix, tws;  // twiddle stride M / (ns radix)
+};
+struct GPlan {
+    int M, H, C, passes;  // C transforms per workgroup
+    FastDiv m, h, c;
+    GPass pass[9];  // 2^9 = 512
+};
+
+// R-point DFT of v in place, natural order.
+template <int R, int S>
+__device__ __forceinline__ void dft_any(float2 (&v)[R], const float2 *tw, int M)
+{
+    if constexpr (R == 2) {
+        const float2 a = v[0], b = v[1];
+        v[0] = make_float2(a.x + b.x, a.y + b.y);
+        v[1] = make_float2(a.x - b.x, a.y - b.y);
+    } else if constexpr (R == 3) {
+        fft3<S>(v[0], v[1], v[2]);
+    } else if constexpr (R == 4) {
+        fft4<S>(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        fft8<S>(v);
+    } else if constexpr (R == 6 || R == 10) {
+        // 2 and Q are coprime: no twiddles between the two stages
+        constexpr int Q = R / 2;
+        float2 a[Q], b[Q];
+#pragma unroll
+        for (int n = 0; n < Q; n++) {
+            const float2 x = v[(2 * n) % R], y = v[(Q + 2 * n) % R];
+            a[n] = make_float2(x.x + y.x, x.y + y.y);
+            b[n] = make_float2(x.x - y.x, x.y - y.y);
+        }
+        dft_any<Q, S>(a, tw, M);
+        dft_any<Q, S>(b, tw, M);
+#pragma unroll
+        for (int k = 0; k < Q; k++) {
+            v[(k * (Q + 1)) % R] = a[k];
+            v[(Q + k * (Q + 1)) % R] = b[k];
+        }
+    } else {
+        // odd prime: X[k], X[R - k] from the sums and differences of x[n], x[R - n]
+        float2 o[R];
+        o[0] = v[0];
+#pragma unroll
+        for (int n = 1; n < R; n++) o[0] = make_float2(o[0].x + v[n].x, o[0].y + v[n].y);
+#pragma unroll
+        for (int k = 1; k <= R / 2; k++) {
+            float2 e = v[0], d = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int n = 1; n <= R / 2; n++) {
+                const float2 w = tw[(M / R) * ((n * k) % R)];  // (cos, sin), the same for all lanes
+                e.x = fmaf(w.x, v[n].x + v[R - n].x, e.x);
+                e.y = fmaf(w.x, v[n].y + v[R - n].y, e.y);
+                d.x = fmaf(w.y, v[n].x - v[R - n].x, d.x);
+                d.y = fmaf(w.y, v[n].y - v[R - n].y, d.y);
+            }
+            const float sg = S > 0 ? 1.f : -1.f;
+            o[k] = make_float2(fmaf(-sg, d.y, e.x), fmaf(sg, d.x, e.y));
+            o[R - k] = make_float2(fmaf(sg, d.y, e.x), fmaf(-sg, d.x, e.y));
+        }
+#pragma unroll
+        for (int k = 0; k < R; k++) v[k] = o[k];
+    }
+}
+
+// One pass over C transforms of x (pitch M), by 256 threads; barriers inside.
+template <int R, int S, int G>
+__device__ __forceinline__ void fft_pass(float2 *x, const float2 *tw, const GPass &p, int M, int C)
+{
+    constexpr int NB = (G + R - 1) / R;  // C M <= 256 G
+    float2 v[NB][R];
+    int o[NB];
+    const unsigned n = p.count.d, total = (unsigned)C * n;
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        const unsigned w = threadIdx.x + 256u * i;
+        o[i] = -1;
+        if (w < total) {
+            const unsigned c = p.count(w), b = w - c * n, blk = p.ns(b), j = b - blk * p.ns.d;
+            const float2 *in = x + c * (unsigned)M + b;
+            v[i][0] = in[0];
+#pragma unroll
+            for (int q = 1; q < R; q++) {
+                const float2 t = tw[j * p.tws * (unsigned)q];
+                v[i][q] = cmulw(in[q * n], t.x, S > 0 ? t.y : -t.y);
+            }
+            dft_any<R, S>(v[i], tw, M);
+            o[i] = (int)(c * (unsigned)M + blk * p.ns.d * (unsigned)R + j);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+        if (o[i] >= 0) {
+#pragma unroll
+            for (int q = 0; q < R; q++) x[o[i] + q * (int)p.ns.d] = v[i][q];
+        }
+    __syncthreads();
+}
+
+// C transforms of x in place, natural order; the data must be visible (a
+// barrier since the stores).
+template <int S, int G>
+__device__ __forceinline__ void fft_any(float2 *x, const float2 *tw, const GPlan &P, int C)
+{
+    for (int i = 0; i < P.passes; i++) {
+        const GPass &p = P.pass[i];
+        switch (p.radix) {
+        case 8: fft_pass<8, S, G>(x, tw, p, P.M, C); break;
+        case 10: fft_pass<10, S, G>(x, tw, p, P.M, C); break;
+        case 6: fft_pass<6, S, G>(x, tw, p, P.M, C); break;
+        case 4: fft_pass<4, S, G>(x, tw, p, P.M, C); break;
+        case 2: fft_pass<2, S, G>(x, tw, p, P.M, C); break;
+        case 3: fft_pass<3, S, G>(x, tw, p, P.M, C); break;
+        case 5: fft_pass<5, S, G>(x, tw, p, P.M, C); break;
+        case 7: fft_pass<7, S, G>(x, tw, p, P.M, C); break;
+        case 11: fft_pass<11, S, G>(x, tw, p, P.M, C); break;
+        default: fft_pass<13, S, G>(x, tw, p, P.M, C); break;
+        }
+    }
+}
+
+__device__ __forceinline__ void load_tw_any(float2 *tw, int M)
+{
+    for (int q = threadIdx.x; q < M; q += 256) {
+        // 2q/M = a + r: the rounding of a is made up to first order
+        const float a = (float)(2 * q) / (float)M, r = (float)M_PI * (fmaf(-a, (float)M, (float)(2 * q)) / (float)M);
+        float sn, cs;
+        sincospif(a, &sn, &cs);
+        tw[q] = make_float2(fmaf(-r, sn, cs), fmaf(r, cs, sn));
+    }
+}
+
+// total items of a workgroup through load and then put, U loads of a thread in
+// flight; the clamped last item may be put several times (the same value).
+template <int U, typename L, typename F>
+__device__ __forceinline__ void g_stage(int total, L load, F put)
+{
+    for (int b = 0; b < total; b += U * 256) {
+        decltype(load(0)) v[U];
+#pragma unroll
+        for (int i = 0; i < U; i++) v[i] = load(min(b + (int)threadIdx.x + 256 * i, total - 1));
+#pragma unroll
+        for (int i = 0; i < U; i++) put(min(b + (int)threadIdx.x + 256 * i, total - 1), v[i]);
+    }
+}
+
+// The four image passes, as k_inv_rows, k_inv_cols, k_fwd_cols and k_fwd_rows
+// have them.  Grid: (ceil(H / C) or ceil(N / 2C), images).
+template <int G>
+__global__ __launch_bounds__(256) void g_inv_rows(const float *__restrict__ cas, float2 *__restrict__ tmp, int n, int N, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2, ky0 = C * (int)blockIdx.x;
+    load_tw_any(tw, M);
+    for (int a = blockIdx.y; a < n; a += gridDim.y) {
+        const float *im = cas + (size_t)a * M * M;
+        g_stage<G>(C * M, [&](int e) {
+            const int c = (int)P.m(e), kx = e - c * M, ky = min(ky0 + c, H - 1);
+            return make_float2(im[ky * M + kx], im[(ky ? M - ky : 0) * M + (kx ? M - kx : 0)]);
+        }, [&](int e, float2 v) {
+            const int c = (int)P.m(e), kx = e - c * M, ky = min(ky0 + c, H - 1);
+            const float sg = chk(kx + ky);
+            x[e] = kx != 0 && ky != 0 ? make_float2(sg * (0.5f * (v.x + v.y)), sg * (0.5f * (v.x - v.y)))
+                                      : make_float2(0.f, 0.f);
+        });
+        __syncthreads();
+        fft_any<1, G>(x, tw, P, C);
+        for (int e = threadIdx.x; e < C * M; e += 256) {
+            const int c = (int)P.m(e), px = e - c * M - off, ky = ky0 + c;
+            if (ky < H && px >= 0 && px < N) tmp[((size_t)a * H + ky) * N + px] = x[e];
+        }
+        __syncthreads();
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_inv_cols(const float2 *__restrict__ tmp, float *__restrict__ imgs, int n, int N,
+                                                  float scale, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2, px0 = 2 * C * (int)blockIdx.x;
+    load_tw_any(tw, M);
+    for (int a = blockIdx.y; a < n; a += gridDim.y) {
+        g_stage<G>(C * H, [&](int e) {  // N is even: columns come in pairs
+            const int ky = (int)P.c(e), c = e - ky * C, p0 = min(px0 + 2 * c, N - 2);
+            const float2 *r = tmp + ((size_t)a * H + ky) * N + p0;
+            return make_float4(r[0].x, r[0].y, r[1].x, r[1].y);
+        }, [&](int e, float4 v) {
+            const int ky = (int)P.c(e), c = e - ky * C;
+            x[c * M + ky] = make_float2(v.x - v.w, v.y + v.z);
+            if (ky != 0 && ky != M / 2) x[c * M + M - ky] = make_float2(v.x + v.w, v.z - v.y);
+        });
+        __syncthreads();
+        fft_any<1, G>(x, tw, P, C);
+        for (int e = threadIdx.x; e < 2 * C * N; e += 256) {
+            const int py = (int)P.c(e >> 1), col = e - py * 2 * C, px = px0 + col, my = py + off;
+            if (px >= N) continue;
+            const float2 z = x[(col >> 1) * M + my];
+            imgs[((size_t)a * N + py) * N + px] = chk(px + off + my) * ((col & 1) ? z.y : z.x) * scale;
+        }
+        __syncthreads();
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_fwd_cols(const float *__restrict__ imgs, float2 *__restrict__ tmp, int n, int N, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2, px0 = 2 * C * (int)blockIdx.x;
+    load_tw_any(tw, M);
+    float *xs = reinterpret_cast<float *>(x);
+    for (int a = blockIdx.y; a < n; a += gridDim.y) {
+        g_stage<G>(2 * C * M, [&](int e) {
+            const int my = (int)P.c(e >> 1), col = e - my * 2 * C, px = px0 + col, py = my - off;
+            return imgs[((size_t)a * N + min(max(py, 0), N - 1)) * N + min(px, N - 1)];
+        }, [&](int e, float raw) {
+            const int my = (int)P.c(e >> 1), col = e - my * 2 * C, px = px0 + col, py = my - off;
+            const bool in = py >= 0 && py < N && px < N;
+            xs[((col >> 1) * M + my) * 2 + (col & 1)] = in ? chk(px + off + my) * raw : 0.f;
+        });
+        __syncthreads();
+        fft_any<-1, G>(x, tw, P, C);
+        for (int e = threadIdx.x; e < 2 * C * H; e += 256) {
+            const int ky = (int)P.c(e >> 1), col = e - ky * 2 * C, px = px0 + col;
+            if (px >= N) continue;
+            const float2 z = x[(col >> 1) * M + ky], zm = x[(col >> 1) * M + (ky ? M - ky : 0)];
+            tmp[((size_t)a * H + ky) * N + px] = (col & 1) ? make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x))
+                                                           : make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));
+        }
+        __syncthreads();
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_fwd_rows(const float2 *__restrict__ tmp, float *__restrict__ cas, int n, int N,
+                                                  float scale, int zeroNyq, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2, ky0 = C * (int)blockIdx.x;
+    load_tw_any(tw, M);
+    for (int a = blockIdx.y; a < n; a += gridDim.y) {
+        g_stage<G>(C * M, [&](int e) {
+            const int c = (int)P.m(e), px = e - c * M - off, ky = min(ky0 + c, H - 1);
+            return tmp[((size_t)a * H + ky) * N + min(max(px, 0), N - 1)];
+        }, [&](int e, float2 raw) {
+            const int c = (int)P.m(e), px = e - c * M - off;
+            x[e] = px >= 0 && px < N ? raw : make_float2(0.f, 0.f);
+        });
+        __syncthreads();
+        fft_any<-1, G>(x, tw, P, C);
+        float *o = cas + (size_t)a * M * M;
+        for (int e = threadIdx.x; e < C * M; e += 256) {
+            const int c = (int)P.m(e), kx = e - c * M, ky = ky0 + c;
+            if (ky >= H) continue;
+            const float2 F = x[e], Fm = x[c * M + (kx ? M - kx : 0)];
+            const float sd = chk(kx + ky);
+            o[ky * M + kx] = (zeroNyq && (kx == 0 || ky == 0)) ? 0.f : (sd * F.x + sd * F.y) * scale;
+            if (ky != 0 && ky != M / 2)  // CAS row M - ky from conj F[ky][(M - kx) % M]
+                o[(M - ky) * M + kx] = (zeroNyq && kx == 0) ? 0.f : (sd * Fm.x - sd * Fm.y) * scale;
+        }
+        __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Volume chains (utils/CASFromVol_Gridder.m:34-60, utils/volFromCAS_Gridder.m:
 // 37-56).  In 3-D the shift identity carries a global sign (-1)^(3M/2).
 // ---------------------------------------------------------------------------
@@ -3108,8 +3391,10 @@ __global__ __launch_bounds__(256) void k_vol_inv_z(const float *__restrict__ cas
 #pragma unroll
     for (int n2 = 0; n2 < R; n2++) {
         const int kz = t + 16 * n2;
-        const float s = (zeroNyq && (kx == 0 || ky == 0 || kz == 0)) ? 0.f : chk(kx + ky + kz);
-        v[n2] = make_float2(s * (0.5f * (c1[n2] + c2[n2])), s * (0.5f * (c1[n2] - c2[n2])));
+        const float s = chk(kx + ky + kz);
+        const bool drop = zeroNyq && (kx == 0 || ky == 0 || kz == 0);  // whatever is there, NaN included
+        v[n2] = drop ? make_float2(0.f, 0.f)
+                     : make_float2(s * (0.5f * (c1[n2] + c2[n2])), s * (0.5f * (c1[n2] - c2[n2])));
     }
     __syncthreads();
     fft_m<R, 1>(v, t, sx + f * G::FFB, tw);
@@ -3162,6 +3447,161 @@ __global__ __launch_bounds__(256) void k_vol_inv_x(const float2 *__restrict__ A,
         const float sg = chk(mx);
         if (row0 < rows) vol[(size_t)row0 * N + px] = sg * s0 * (float)(w * w0 * (double)z.x);
         if (row0 + 1 < rows) vol[(size_t)(row0 + 1) * N + px] = sg * s1 * (float)(w * w1 * (double)z.y);
+    }
+}
+
+// The volume passes for the other sizes (fft_any).  Along y and z a workgroup
+// takes C neighbouring kx of one line.
+__device__ __forceinline__ VolLine g_vol_line(int n, int tiles, int C)
+{
+    const int idx = (int)(blockIdx.x >> 3), q = idx / tiles;
+    const int line = q * 8 + (int)(blockIdx.x & 7u);
+    return {line, C * (idx - q * tiles), line < n};
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_vol_fwd_x(const float *__restrict__ vol, int N, float2 *__restrict__ A,
+                                                   const float *__restrict__ pc, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2, rows = N * N, row0 = 2 * C * (int)blockIdx.x;
+    load_tw_any(tw, M);
+    float *xs = reinterpret_cast<float *>(x);
+    g_stage<G>(2 * C * M, [&](int e) {
+        const int r = (int)P.m(e), mx = e - r * M, row = min(row0 + r, rows - 1);
+        return vol[(size_t)row * N + min(max(mx - off, 0), N - 1)];
+    }, [&](int e, float raw) {
+        const int r = (int)P.m(e), mx = e - r * M, q = mx - off, row = min(row0 + r, rows - 1);
+        const int mz = row / N + off, my = row % N + off;
+        const double w = (double)pc[mx] * (double)pc[my] * (double)pc[mz];
+        xs[((r >> 1) * M + mx) * 2 + (r & 1)] = q >= 0 && q < N ? chk(mx + my + mz) * (float)(w * (double)raw) : 0.f;
+    });
+    __syncthreads();
+    fft_any<-1, G>(x, tw, P, C);
+    for (int e = threadIdx.x; e < 2 * C * H; e += 256) {
+        const int r = (int)P.h(e), k = e - r * H, row = row0 + r;
+        if (row >= rows) break;
+        const float2 z = x[(r >> 1) * M + k], zm = x[(r >> 1) * M + (k ? M - k : 0)];
+        A[(size_t)row * H + k] = (r & 1) ? make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x))
+                                         : make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));
+    }
+}
+
+template <int S, int G>
+__global__ __launch_bounds__(256) void g_vol_y(const float2 *__restrict__ in, float2 *__restrict__ out, int N, int tiles, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2;
+    load_tw_any(tw, M);
+    const VolLine l = g_vol_line(N, tiles, C);
+    if (!l.ok) return;  // uniform
+    const int nIn = S < 0 ? N : M, oIn = S < 0 ? off : 0, nOut = S < 0 ? M : N, oOut = S < 0 ? 0 : off;
+    g_stage<G>(C * M, [&](int e) {
+        const int my = (int)P.c(e), c = e - my * C, y = my - oIn;
+        return in[((size_t)l.line * nIn + min(max(y, 0), nIn - 1)) * H + min(l.kx0 + c, H - 1)];
+    }, [&](int e, float2 raw) {
+        const int my = (int)P.c(e), c = e - my * C, y = my - oIn;
+        x[c * M + my] = y >= 0 && y < nIn ? raw : make_float2(0.f, 0.f);
+    });
+    __syncthreads();
+    fft_any<S, G>(x, tw, P, C);
+    for (int e = threadIdx.x; e < C * nOut; e += 256) {
+        const int y = (int)P.c(e), c = e - y * C;
+        if (l.kx0 + c < H) out[((size_t)l.line * nOut + y) * H + l.kx0 + c] = x[c * M + y + oOut];
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_vol_fwd_z(const float2 *__restrict__ B, int N, float *__restrict__ casVol, int V,
+                                                   int pad, float gsign, int tiles, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2;
+    load_tw_any(tw, M);
+    const VolLine l = g_vol_line(M, tiles, C);
+    if (!l.ok) return;  // uniform
+    const int ky = l.line, my = ky ? M - ky : 0;
+    g_stage<G>(C * M, [&](int e) {
+        const int mz = (int)P.c(e), c = e - mz * C, z = mz - off;
+        return B[((size_t)min(max(z, 0), N - 1) * M + ky) * H + min(l.kx0 + c, H - 1)];
+    }, [&](int e, float2 raw) {
+        const int mz = (int)P.c(e), c = e - mz * C, z = mz - off;
+        x[c * M + mz] = z >= 0 && z < N ? raw : make_float2(0.f, 0.f);
+    });
+    __syncthreads();
+    fft_any<-1, G>(x, tw, P, C);
+    for (int e = threadIdx.x; e < C * M; e += 256) {
+        const int kz = (int)P.c(e), c = e - kz * C, kx = l.kx0 + c;
+        if (kx >= H) continue;
+        const float2 F = x[c * M + kz];
+        const float s = gsign * chk(kx + ky + kz);
+        casVol[((size_t)(kz + pad) * V + (ky + pad)) * V + (kx + pad)] = s * F.x + s * F.y;
+        if (kx != 0 && kx != M / 2)
+            casVol[((size_t)((kz ? M - kz : 0) + pad) * V + (my + pad)) * V + (M - kx + pad)] = s * F.x - s * F.y;
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_vol_inv_z(const float *__restrict__ casVol, int V, int pad, float2 *__restrict__ B,
+                                                   int N, int zeroNyq, int tiles, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2;
+    load_tw_any(tw, M);
+    const VolLine l = g_vol_line(M, tiles, C);
+    if (!l.ok) return;  // uniform
+    const int ky = l.line, my = ky ? M - ky : 0;
+    g_stage<G>(C * M, [&](int e) {
+        const int kz = (int)P.c(e), c = e - kz * C, kx = min(l.kx0 + c, H - 1);
+        return make_float2(casVol[((size_t)(kz + pad) * V + (ky + pad)) * V + (kx + pad)],
+                           casVol[((size_t)((kz ? M - kz : 0) + pad) * V + (my + pad)) * V + ((kx ? M - kx : 0) + pad)]);
+    }, [&](int e, float2 v) {
+        const int kz = (int)P.c(e), c = e - kz * C, kx = min(l.kx0 + c, H - 1);
+        const float c1 = v.x, c2 = v.y, s = chk(kx + ky + kz);
+        const bool drop = zeroNyq && (kx == 0 || ky == 0 || kz == 0);  // whatever is there, NaN included
+        x[c * M + kz] = drop ? make_float2(0.f, 0.f) : make_float2(s * (0.5f * (c1 + c2)), s * (0.5f * (c1 - c2)));
+    });
+    __syncthreads();
+    fft_any<1, G>(x, tw, P, C);
+    for (int e = threadIdx.x; e < C * N; e += 256) {
+        const int z = (int)P.c(e), c = e - z * C;
+        if (l.kx0 + c < H) B[((size_t)z * M + ky) * H + l.kx0 + c] = x[c * M + z + off];
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void g_vol_inv_x(const float2 *__restrict__ A, float *__restrict__ vol, int N,
+                                                   const float *__restrict__ pc, double scale, GPlan P)
+{
+    __shared__ float2 x[256 * G];
+    __shared__ float2 tw[512];
+    const int M = P.M, H = P.H, C = P.C, off = (M - N) / 2, rows = N * N, row0 = 2 * C * (int)blockIdx.x;
+    load_tw_any(tw, M);
+    g_stage<G>(C * H, [&](int e) {
+        const int c = (int)P.h(e), k = e - c * H;
+        const float2 p = A[(size_t)min(row0 + 2 * c, rows - 1) * H + k], q = A[(size_t)min(row0 + 2 * c + 1, rows - 1) * H + k];
+        return make_float4(p.x, p.y, q.x, q.y);
+    }, [&](int e, float4 v) {
+        const int c = (int)P.h(e), k = e - c * H;
+        const float2 p = make_float2(v.x, v.y), q = make_float2(v.z, v.w);
+        // a real transform has no imaginary part at k = 0 and M/2
+        const bool real = k == 0 || k == M / 2;
+        x[c * M + k] = real ? make_float2(p.x, q.x) : make_float2(p.x - q.y, p.y + q.x);
+        if (!real) x[c * M + M - k] = make_float2(p.x + q.y, q.x - p.y);
+    });
+    __syncthreads();
+    fft_any<1, G>(x, tw, P, C);
+    for (int e = threadIdx.x; e < 2 * C * M; e += 256) {
+        const int r = (int)P.m(e), mx = e - r * M, px = mx - off, row = row0 + r;
+        if (px < 0 || px >= N || row >= rows) continue;
+        const int mz = row / N + off, my = row % N + off;
+        const float2 z = x[(r >> 1) * M + mx];
+        const double w = (double)pc[mx] * (double)pc[my] * (double)pc[mz] * scale;
+        vol[(size_t)row * N + px] = chk(mx + my + mz) * (float)(w * (double)((r & 1) ? z.y : z.x));
     }
 }
 
@@ -3890,6 +4330,70 @@ bool fused_chain_supported(int M, int N)
     return (M == 128 || M == 192 || M == 256 || M == 384 || M == 512) && N >= 1 && N <= M;
 }
 
+// Radices of M for fft_any; false when M has a prime factor beyond 13, is odd
+// or does not fit.  Factors 2 that do not make up an 8 go with a 5 or a 3.
+static bool g_plan(int M, GPlan &P)
+{
+    if (M < 2 || M % 2 || M > 512) return false;
+    P.M = M;
+    P.H = M / 2 + 1;
+    P.m.set((unsigned)M);
+    P.h.set((unsigned)P.H);
+    P.passes = 0;
+    int left = M;
+    unsigned ns = 1;
+    const auto take = [&](unsigned r) {
+        GPass &p = P.pass[P.passes++];
+        p.radix = r;
+        p.ns.set(ns);
+        p.count.set((unsigned)M / r);
+        ns *= r;
+        p.tws = (unsigned)M / ns;
+        left /= (int)r;
+    };
+    const auto twos = [&] {
+        int n = 0;
+        while (left % (2 << n) == 0) n++;
+        return n % 3;
+    };
+    for (unsigned r : {10u, 6u})
+        while (left % (int)r == 0 && twos()) take(r);
+    for (unsigned r : {8u, 4u, 2u, 3u, 5u, 7u, 11u, 13u})
+        while (left % (int)r == 0) take(r);
+    return left == 1;
+}
+
+// Values a thread holds in fft_any (G) and the transforms of a workgroup (C M
+// <= 256 G, at most 16) for n lines, reps times.  The kernels are as long as G
+// and a short launch waits for its instructions: 4 while 8 would leave the
+// card with less than four workgroups per CU (one image of M = 240: 17.9 us
+// with 16, 13.2 with 4; 300 images of M = 200: 58 with 16, 48 with 8; of M =
+// 480: 218 with 8, 282 with 4).
+static int g_split(GPlan &P, int n, size_t reps, unsigned &groups)
+{
+    int most = 0, G = 8;
+    for (;; G = 4) {
+        most = std::min(16, 256 * G / P.M);
+        if (G == 4 || (size_t)((n + most - 1) / most) * reps >= 1024) break;
+    }
+    const int even = (n + most - 1) / most;
+    P.C = (n + even - 1) / even;
+    P.c.set((unsigned)P.C);
+    groups = (unsigned)((n + P.C - 1) / P.C);
+    return G;
+}
+#define MGG_G(G, kernel, kernel8, ...)                              \
+    do {                                                            \
+        if ((G) == 4) hipLaunchKernelGGL((kernel), __VA_ARGS__);    \
+        else hipLaunchKernelGGL((kernel8), __VA_ARGS__);            \
+    } while (0)
+
+bool image_chain_supported(int M, int N)
+{
+    GPlan P;
+    return N >= 1 && N <= M && (fused_chain_supported(M, N) || ((M - N) % 2 == 0 && g_plan(M, P)));  // N even
+}
+
 template <int R>
 static void fused_inverse(const float *cas, float2 *tmp, float *imgs, int N, int n, float scale, hipStream_t s)
 {
@@ -3914,7 +4418,18 @@ hipError_t launch_fused_cas_to_images(const float *cas, float2 *tmp, float *imgs
                                       float scale, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    if (!fused_chain_supported(M, N)) return hipErrorInvalidValue;
+    if (!image_chain_supported(M, N)) return hipErrorInvalidValue;
+    if (!fused_chain_supported(M, N)) {
+        GPlan P;
+        if (!g_plan(M, P)) return hipErrorInvalidValue;
+        const unsigned ny = (unsigned)std::min(n, 65535);
+        unsigned groups = 0;
+        int G = g_split(P, P.H, (size_t)n, groups);
+        MGG_G(G, (g_inv_rows<4>), (g_inv_rows<8>), dim3(groups, ny), dim3(256), 0, s, cas, tmp, n, N, P);
+        G = g_split(P, N / 2, (size_t)n, groups);
+        MGG_G(G, (g_inv_cols<4>), (g_inv_cols<8>), dim3(groups, ny), dim3(256), 0, s, tmp, imgs, n, N, scale, P);
+        return hipGetLastError();
+    }
     switch (M) {
     case 128: fused_inverse<8>(cas, tmp, imgs, N, n, scale, s); break;
     case 192: fused_inverse<12>(cas, tmp, imgs, N, n, scale, s); break;
@@ -3929,7 +4444,18 @@ hipError_t launch_fused_images_to_cas(const float *imgs, float2 *tmp, float *cas
                                       float scale, int zeroNyq, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    if (!fused_chain_supported(M, N)) return hipErrorInvalidValue;
+    if (!image_chain_supported(M, N)) return hipErrorInvalidValue;
+    if (!fused_chain_supported(M, N)) {
+        GPlan P;
+        if (!g_plan(M, P)) return hipErrorInvalidValue;
+        const unsigned ny = (unsigned)std::min(n, 65535);
+        unsigned groups = 0;
+        int G = g_split(P, N / 2, (size_t)n, groups);
+        MGG_G(G, (g_fwd_cols<4>), (g_fwd_cols<8>), dim3(groups, ny), dim3(256), 0, s, imgs, tmp, n, N, P);
+        G = g_split(P, P.H, (size_t)n, groups);
+        MGG_G(G, (g_fwd_rows<4>), (g_fwd_rows<8>), dim3(groups, ny), dim3(256), 0, s, tmp, cas, n, N, scale, zeroNyq, P);
+        return hipGetLastError();
+    }
     switch (M) {
     case 128: fused_forward<8>(imgs, tmp, cas, N, n, scale, zeroNyq, s); break;
     case 192: fused_forward<12>(imgs, tmp, cas, N, n, scale, zeroNyq, s); break;
@@ -3943,7 +4469,10 @@ hipError_t launch_fused_images_to_cas(const float *imgs, float2 *tmp, float *cas
 bool fused_volume_supported(int M, int N)
 {
     // B (N M H complex) has to fit the M^3 real scratch
-    return fused_chain_supported(M, N) && N % 2 == 0 && (size_t)N * (M + 2) <= (size_t)M * M;
+    // Below M = 80 one rocFFT plan's few launches are as fast or faster than
+    // the general passes (M = 64: 17 us against 18; 80: 42 against 39 there and
+    // back; 100: 71 against 41).
+    return image_chain_supported(M, N) && M >= 80 && N % 2 == 0 && (size_t)N * (M + 2) <= (size_t)M * M;
 }
 
 template <int R>
@@ -3975,6 +4504,21 @@ hipError_t launch_fused_volume_to_cas(const float *vol, int N, float *casVol, in
     if (!fused_volume_supported(M, N)) return hipErrorInvalidValue;
     const float g = ((3 * (M / 2)) & 1) ? -1.f : 1.f;
     const int V = M + 2 * pad;
+    if (!fused_chain_supported(M, N)) {
+        GPlan P;
+        if (!g_plan(M, P)) return hipErrorInvalidValue;
+        unsigned T = 0;
+        int G = g_split(P, N * N / 2, 1, T);
+        MGG_G(G, (g_vol_fwd_x<4>), (g_vol_fwd_x<8>), dim3(T), dim3(256), 0, s, vol, N, a, precomp, P);
+        G = g_split(P, P.H, (size_t)N, T);
+        MGG_G(G, (g_vol_y<-1, 4>), (g_vol_y<-1, 8>), dim3((unsigned)(N + 7) / 8 * 8 * T), dim3(256), 0, s, a, b, N,
+              (int)T, P);
+        if (pad > 0) hipLaunchKernelGGL(k_casvol_shell, dim3((unsigned)V, 8), dim3(256), 0, s, casVol, V, pad);
+        G = g_split(P, P.H, (size_t)M, T);
+        MGG_G(G, (g_vol_fwd_z<4>), (g_vol_fwd_z<8>), dim3((unsigned)(M + 7) / 8 * 8 * T), dim3(256), 0, s, b, N, casVol, V,
+              pad, g, (int)T, P);
+        return hipGetLastError();
+    }
     switch (M) {
     case 128: fused_vol_fwd<8>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
     case 192: fused_vol_fwd<12>(vol, N, casVol, V, pad, precomp, a, b, g, s); break;
@@ -3991,6 +4535,20 @@ hipError_t launch_fused_cas_to_volume(const float *casVol, int M, int pad, float
     if (!fused_volume_supported(M, N)) return hipErrorInvalidValue;
     const double sc = (((3 * (M / 2)) & 1) ? -1.0 : 1.0) * (double)scale;
     const int V = M + 2 * pad;
+    if (!fused_chain_supported(M, N)) {
+        GPlan P;
+        if (!g_plan(M, P)) return hipErrorInvalidValue;
+        unsigned T = 0;
+        int G = g_split(P, P.H, (size_t)M, T);
+        MGG_G(G, (g_vol_inv_z<4>), (g_vol_inv_z<8>), dim3((unsigned)(M + 7) / 8 * 8 * T), dim3(256), 0, s, casVol, V, pad, b, N,
+              zeroNyquist, (int)T, P);
+        G = g_split(P, P.H, (size_t)N, T);
+        MGG_G(G, (g_vol_y<1, 4>), (g_vol_y<1, 8>), dim3((unsigned)(N + 7) / 8 * 8 * T), dim3(256), 0, s, b, a, N,
+              (int)T, P);
+        G = g_split(P, N * N / 2, 1, T);
+        MGG_G(G, (g_vol_inv_x<4>), (g_vol_inv_x<8>), dim3(T), dim3(256), 0, s, a, vol, N, precomp, sc, P);
+        return hipGetLastError();
+    }
     switch (M) {
     case 128: fused_vol_inv<8>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;
     case 192: fused_vol_inv<12>(casVol, V, pad, vol, N, precomp, a, b, zeroNyquist, sc, s); break;

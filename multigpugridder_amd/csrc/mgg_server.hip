@@ -428,7 +428,7 @@ struct mgg_server {
                 float *out = dImgs + b.imgBase[pc.seg] + (size_t)(pc.lo - sg.offset) * nn;
                 for (int a0 = 0; a0 < n; a0 += (int)kFftBatch) {
                     const int gN = std::min((int)kFftBatch, n - a0);
-                    if (fused_chain_supported(M, N)) {
+                    if (image_chain_supported(M, N)) {
                         check_launch(launch_fused_cas_to_images(cas + a0 * mm, dHerm, out + a0 * nn, M, N, gN, scale,
                                                                 p.stream),
                                      "fused_cas_to_images");
@@ -501,7 +501,7 @@ struct mgg_server {
             // forward image chain (ImgsToCASImgs), groups of kFftBatch images
             for (int a0 = 0; a0 < cnt; a0 += (int)kFftBatch) {
                 const int gN = std::min((int)kFftBatch, cnt - a0);
-                if (fused_chain_supported(M, N)) {
+                if (image_chain_supported(M, N)) {
                     check_launch(launch_fused_images_to_cas(imgs + a0 * nn, dHerm, dCas + a0 * mm, M, N, gN, 1.0f, 0,
                                                             p.stream),
                                  "fused_images_to_cas");

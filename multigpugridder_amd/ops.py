@@ -257,8 +257,9 @@ def back_project_adjoint(cas_images: torch.Tensor, axes: torch.Tensor, v: int, m
 
 def cas_images_to_images(cas_images: torch.Tensor, n: int, out: torch.Tensor | None = None,
                          clobber: bool = False) -> torch.Tensor:
-    """(P, m, m) CAS images -> (P, n, n) images.  The kernel uses its input as
-    scratch; unless ``clobber`` it works on a copy."""
+    """(P, m, m) CAS images -> (P, n, n) images.  Where the chain uses its input
+    as scratch (m with a prime factor beyond 13 or above 512), or ``out`` shares
+    memory with it, it works on a copy unless ``clobber``."""
     p, m = _stack_edge(cas_images, "cas_images")
     if not 0 < n <= m:
         raise ValueError(f"image size n must be in [1, {m}], got {n}")
@@ -266,9 +267,12 @@ def cas_images_to_images(cas_images: torch.Tensor, n: int, out: torch.Tensor | N
         _need_numel(out, p * n * n, "out")
     _same_device(("cas_images", cas_images), ("out", out))
     _check(cas_images, "cas_images")
-    src = cas_images if clobber else cas_images.clone()
     if out is None:
         out = torch.empty((p, n, n), device=cas_images.device, dtype=torch.float32)
+        shared = False
+    else:
+        shared = out.untyped_storage().data_ptr() == cas_images.untyped_storage().data_ptr()
+    src = cas_images if clobber or (not shared and _lib.image_chain_reads_only(m, n)) else cas_images.clone()
     _check(out, "out")
     _lib.call("mgg_op_cas_images_to_images", _ptr(src), _ptr(out), p, m, n, _stream())
     return out
