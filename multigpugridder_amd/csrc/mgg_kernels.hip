@@ -2844,7 +2844,9 @@ struct GPlan {
     GPass pass[9];  // 2^9 = 512
 };
 
-// R-point DFT of v in place, natural order.
+// R-point DFT of v in place, natural order.  The second halves of the
+// constants of 3 and 5 keep their rounding out of the result (M = 100, there
+// and back: 1.27e-7 and 1.36e-7 against 1.45e-7 and 1.47e-7 without).
 template <int R, int S>
 __device__ __forceinline__ void dft_any(float2 (&v)[R], const float2 *tw, int M)
 {
@@ -2853,7 +2855,14 @@ __device__ __forceinline__ void dft_any(float2 (&v)[R], const float2 *tw, int M)
         v[0] = make_float2(a.x + b.x, a.y + b.y);
         v[1] = make_float2(a.x - b.x, a.y - b.y);
     } else if constexpr (R == 3) {
-        fft3<S>(v[0], v[1], v[2]);
+        constexpr float c = 0.866025403784438647f, c2 = (float)(0.866025403784438647 - (double)c);
+        const float sg = S > 0 ? 1.f : -1.f;
+        const float2 t = make_float2(v[1].x + v[2].x, v[1].y + v[2].y), u = make_float2(v[1].x - v[2].x, v[1].y - v[2].y);
+        const float2 e = make_float2(fmaf(-0.5f, t.x, v[0].x), fmaf(-0.5f, t.y, v[0].y));
+        const float2 f = make_float2(sg * fmaf(c, u.x, c2 * u.x), sg * fmaf(c, u.y, c2 * u.y));
+        v[0] = make_float2(v[0].x + t.x, v[0].y + t.y);
+        v[1] = make_float2(e.x - f.y, e.y + f.x);
+        v[2] = make_float2(e.x + f.y, e.y - f.x);
     } else if constexpr (R == 4) {
         fft4<S>(v[0], v[1], v[2], v[3]);
     } else if constexpr (R == 8) {
@@ -2875,23 +2884,50 @@ __device__ __forceinline__ void dft_any(float2 (&v)[R], const float2 *tw, int M)
             v[(k * (Q + 1)) % R] = a[k];
             v[(Q + k * (Q + 1)) % R] = b[k];
         }
+    } else if constexpr (R == 5) {
+        // cos 72 and cos 144 degrees are -1/4 +- sqrt(5)/4
+        constexpr float q = 0.559016994374947424f, q2 = (float)(0.559016994374947424 - (double)q);
+        constexpr float s1 = 0.951056516295153572f, s12 = (float)(0.951056516295153572 - (double)s1);
+        constexpr float s2 = 0.587785252292473129f, s22 = (float)(0.587785252292473129 - (double)s2);
+        const float2 t1 = make_float2(v[1].x + v[4].x, v[1].y + v[4].y), t2 = make_float2(v[2].x + v[3].x, v[2].y + v[3].y);
+        const float2 t3 = make_float2(v[1].x - v[4].x, v[1].y - v[4].y), t4 = make_float2(v[2].x - v[3].x, v[2].y - v[3].y);
+        const float2 m = make_float2(t1.x + t2.x, t1.y + t2.y), d = make_float2(t1.x - t2.x, t1.y - t2.y);
+        const float2 a = make_float2(fmaf(-0.25f, m.x, v[0].x), fmaf(-0.25f, m.y, v[0].y));
+        const float2 b = make_float2(fmaf(q2, d.x, q * d.x), fmaf(q2, d.y, q * d.y));
+        const float sg = S > 0 ? 1.f : -1.f;
+        const float2 e1 = make_float2(a.x + b.x, a.y + b.y), e2 = make_float2(a.x - b.x, a.y - b.y);
+        const float2 f1 = make_float2(sg * fmaf(s1, t3.x, fmaf(s2, t4.x, fmaf(s12, t3.x, s22 * t4.x))),
+                                      sg * fmaf(s1, t3.y, fmaf(s2, t4.y, fmaf(s12, t3.y, s22 * t4.y))));
+        const float2 f2 = make_float2(sg * fmaf(s2, t3.x, fmaf(-s1, t4.x, fmaf(s22, t3.x, -s12 * t4.x))),
+                                      sg * fmaf(s2, t3.y, fmaf(-s1, t4.y, fmaf(s22, t3.y, -s12 * t4.y))));
+        v[0] = make_float2(v[0].x + m.x, v[0].y + m.y);
+        v[1] = make_float2(e1.x - f1.y, e1.y + f1.x);
+        v[4] = make_float2(e1.x + f1.y, e1.y - f1.x);
+        v[2] = make_float2(e2.x - f2.y, e2.y + f2.x);
+        v[3] = make_float2(e2.x + f2.y, e2.y - f2.x);
     } else {
         // odd prime: X[k], X[R - k] from the sums and differences of x[n], x[R - n]
-        float2 o[R];
-        o[0] = v[0];
+        float2 o[R], p[R / 2], m[R / 2];
+        o[0] = make_float2(0.f, 0.f);
 #pragma unroll
-        for (int n = 1; n < R; n++) o[0] = make_float2(o[0].x + v[n].x, o[0].y + v[n].y);
+        for (int n = 1; n <= R / 2; n++) {
+            p[n - 1] = make_float2(v[n].x + v[R - n].x, v[n].y + v[R - n].y);
+            m[n - 1] = make_float2(v[n].x - v[R - n].x, v[n].y - v[R - n].y);
+            o[0] = make_float2(o[0].x + p[n - 1].x, o[0].y + p[n - 1].y);
+        }
+        o[0] = make_float2(v[0].x + o[0].x, v[0].y + o[0].y);
 #pragma unroll
         for (int k = 1; k <= R / 2; k++) {
-            float2 e = v[0], d = make_float2(0.f, 0.f);
+            float2 e = make_float2(0.f, 0.f), d = make_float2(0.f, 0.f);
 #pragma unroll
             for (int n = 1; n <= R / 2; n++) {
                 const float2 w = tw[(M / R) * ((n * k) % R)];  // (cos, sin), the same for all lanes
-                e.x = fmaf(w.x, v[n].x + v[R - n].x, e.x);
-                e.y = fmaf(w.x, v[n].y + v[R - n].y, e.y);
-                d.x = fmaf(w.y, v[n].x - v[R - n].x, d.x);
-                d.y = fmaf(w.y, v[n].y - v[R - n].y, d.y);
+                e.x = fmaf(w.x, p[n - 1].x, e.x);
+                e.y = fmaf(w.x, p[n - 1].y, e.y);
+                d.x = fmaf(w.y, m[n - 1].x, d.x);
+                d.y = fmaf(w.y, m[n - 1].y, d.y);
             }
+            e = make_float2(v[0].x + e.x, v[0].y + e.y);  // last: a rounding of v[0] less per term
             const float sg = S > 0 ? 1.f : -1.f;
             o[k] = make_float2(fmaf(-sg, d.y, e.x), fmaf(sg, d.x, e.y));
             o[R - k] = make_float2(fmaf(sg, d.y, e.x), fmaf(-sg, d.x, e.y));
@@ -4388,6 +4424,14 @@ static int g_split(GPlan &P, int n, size_t reps, unsigned &groups)
         else hipLaunchKernelGGL((kernel8), __VA_ARGS__);            \
     } while (0)
 
+// Whether an image chain takes k_inv_rows and its like.  Their threads hold M /
+// 16 values and the lines beside the cropped images cost them as much as any:
+// at M = 384 and 512 the general passes are faster up to about N = 5/8 M (M =
+// 512, there and back: N = 256 300 images 473 -> 423 us, 16 61 -> 53, one 40 ->
+// 25; N = 512 300 images 758 against 790; M = 384: N = 192 16 images 39.9
+// against 39.2, N = 288 44.7 against 46.4).
+static bool own_image_passes(int M, int N) { return fused_chain_supported(M, N) && (M < 384 || 8 * N > 5 * M); }
+
 bool image_chain_supported(int M, int N)
 {
     GPlan P;
@@ -4419,7 +4463,7 @@ hipError_t launch_fused_cas_to_images(const float *cas, float2 *tmp, float *imgs
 {
     if (n <= 0) return hipSuccess;
     if (!image_chain_supported(M, N)) return hipErrorInvalidValue;
-    if (!fused_chain_supported(M, N)) {
+    if (!own_image_passes(M, N)) {
         GPlan P;
         if (!g_plan(M, P)) return hipErrorInvalidValue;
         const unsigned ny = (unsigned)std::min(n, 65535);
@@ -4445,7 +4489,7 @@ hipError_t launch_fused_images_to_cas(const float *imgs, float2 *tmp, float *cas
 {
     if (n <= 0) return hipSuccess;
     if (!image_chain_supported(M, N)) return hipErrorInvalidValue;
-    if (!fused_chain_supported(M, N)) {
+    if (!own_image_passes(M, N)) {
         GPlan P;
         if (!g_plan(M, P)) return hipErrorInvalidValue;
         const unsigned ny = (unsigned)std::min(n, 65535);

@@ -35,12 +35,13 @@ def _inv(cas, n, dims, drop):
     return x
 
 
-# every radix alone and together, the smallest sizes, one and two workgroups of
+# every radix alone and together, both sides of the rule of M = 384 and 512, the smallest sizes, one and two workgroups of
 # lines, 8 transforms per workgroup, a batch beyond one scratch (image_batch),
 # and rocFFT's (factor 17; 514)
 @pytest.mark.parametrize("p,n,m", [(1, 2, 2), (3, 2, 6), (2, 8, 16), (5, 6, 22), (3, 14, 26), (3, 30, 30), (7, 50, 98),
                                    (300, 98, 100), (3, 50, 100), (2, 64, 128), (3, 154, 154), (2, 100, 250), (2, 128, 260), (2, 364, 364),
-                                   (2, 242, 486), (2, 250, 500), (2, 2, 512), (2, 20, 34), (2, 256, 514)])
+                                   (2, 242, 486), (2, 250, 500), (2, 2, 512), (2, 20, 34), (2, 256, 514),
+                                   (2, 240, 384), (2, 242, 384), (2, 320, 512), (2, 322, 512)])
 def test_image_chains(cuda, p, n, m):
     import torch
 
