@@ -332,16 +332,31 @@ const int *brick_order(const ProjGeom &g, int depth, int &len)
     if (!bp_uses_fast_path(g)) return nullptr;
     len = bp_brick_count(g.V, depth);
     std::lock_guard<std::mutex> lk(g_order_mu);
-    auto &b = g_order[std::make_tuple(current_device(), g.V, depth)];
-    if (!b) {
-        std::vector<int> host(len);
-        bp_brick_order(g.V, depth, host.data());
-        auto nb = std::make_unique<DevBuf>();
-        nb->reserve(sizeof(int) * len);
-        HIP_TRY(hipMemcpy(nb->ptr, host.data(), sizeof(int) * len, hipMemcpyHostToDevice));
-        b = std::move(nb);
+    const auto key = std::make_tuple(current_device(), g.V, depth);
+    const auto it = g_order.find(key);
+    if (it != g_order.end()) return it->second->as<int>();
+    std::vector<int> host(len);
+    bp_brick_order(g.V, depth, host.data());
+    auto nb = std::make_unique<DevBuf>();
+    nb->reserve(sizeof(int) * len);
+    HIP_TRY(hipMemcpy(nb->ptr, host.data(), sizeof(int) * len, hipMemcpyHostToDevice));
+    return (g_order[key] = std::move(nb))->as<int>();
+}
+
+// Whether the columns' table can be had: it is made on first use, which a
+// stream under capture cannot do; the call then takes the bricks alone.
+static bool columns_ready(const ProjGeom &g, ColKind kind, hipStream_t s)
+{
+    {
+        std::lock_guard<std::mutex> lk(g_order_mu);
+        if (g_order.count(std::make_tuple(current_device(), g.V, col_depth(kind)))) return true;
     }
-    return b->as<int>();
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st == hipStreamCaptureStatusNone;
 }
 
 hipError_t back_project_launch(float *vol, float *dens, const ProjGeom &g, const float *axes, int n,
@@ -350,7 +365,7 @@ hipError_t back_project_launch(float *vol, float *dens, const ProjGeom &g, const
     int len = 0;
     const int *order = brick_order(g, 8, len);
     const ColKind kind = ColKind::Back;
-    const bool columns = check != nullptr && dens == nullptr && uses_columns(g, n, kind);
+    const bool columns = check != nullptr && dens == nullptr && uses_columns(g, n, kind) && columns_ready(g, kind, s);
     if (columns) {
         int colLen = 0;
         const int *colOrder = brick_order(g, col_depth(kind), colLen);
@@ -364,7 +379,7 @@ hipError_t back_project_launch(float *vol, float *dens, const ProjGeom &g, const
 hipError_t back_project_adjoint_launch(float *vol, const ProjGeom &g, const float *axes, int n, const float *casImgs,
                                        hipStream_t s, const unsigned *finite, unsigned *check)
 {
-    if (check == nullptr || !uses_columns(g, n, ColKind::Adjoint)) {
+    if (check == nullptr || !uses_columns(g, n, ColKind::Adjoint) || !columns_ready(g, ColKind::Adjoint, s)) {
         if (finite == nullptr && check != nullptr) {
             const hipError_t e = launch_check_volume(casImgs, DT_F32, (size_t)std::max(n, 0) * g.M * g.M, g.ker, g.K,
                                                      check, s);
