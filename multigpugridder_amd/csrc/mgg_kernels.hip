@@ -16,6 +16,7 @@
 //
 // Layout: column-major, x fastest.  vol[x + y*V + z*V*V];
 // CAS image a: img[a*M*M + i + j*M]; a direction is 9 floats [u; v; n].
+#include "mgg_columns.h"
 #include "mgg_internal.h"
 
 #include <hip/hip_fp16.h>
@@ -1732,12 +1733,6 @@ __global__ __launch_bounds__(64 * BFW) void bp_fast_kernel(BPArgs p)
 // loop 7.4.
 // ---------------------------------------------------------------------------
 constexpr int BCN = 8;                        // columns per block edge
-enum : int { COL_BACK = 0, COL_ADJOINT = 1 };
-// Index range of the pair table (swept over 200,000 frames, half of them with
-// the normal near a diagonal: -566 to 1,189 for columns of up to six slab
-// voxels, -787 to 1,401 for up to ten transposed ones).
-constexpr int ct_lo(int mode) { return mode == COL_BACK ? -576 : -800; }
-constexpr int ct_hi(int mode) { return mode == COL_BACK ? 1200 : 1416; }
 // Voxels of a block along its columns: four (transpose: three) workgroups of
 // four waves per CU.
 constexpr int bc_depth(int mode) { return mode == COL_BACK ? 24 : 32; }
@@ -1833,7 +1828,7 @@ struct ColVisit {
             const float dj = (float)((ln & 15) - 8);
             float hi = 7.f;
             auto bound = [&](float u, float v) {
-                const float L = 2.02f + 0.5f * (fabsf(u) + fabsf(v));
+                const float L = col_list_reach(u, v);
                 if (fabsf(u) < 1e-6f) {
                     if (fabsf(v * dj) > L) hi = -9.f;
                 } else {
@@ -1892,8 +1887,7 @@ struct ColVisit {
             }
         };
         // only the longest columns reach past the table's ends
-        constexpr bool LONG = GATE ? K == 7 : K > 10;
-        auto clampC = [](int i) { return LONG ? min(max(i, ct_lo(MODE)), ct_hi(MODE) - 1) : i; };
+        auto clampC = [](int i) { return col_clamps(MODE, K) ? min(max(i, ct_lo(MODE)), ct_hi(MODE) - 1) : i; };
         float Ba, Bb, Bc;
         unsigned eff[GATE ? K : 1];
         // NP pixels of the current row from offset di on (bit di + 8 of eff).
@@ -1939,9 +1933,6 @@ struct ColVisit {
                 }
             }
         };
-        using One = std::integral_constant<int, 1>;
-        using Two = std::integral_constant<int, 2>;
-        using Three = std::integral_constant<int, 3>;
         // The next row's first six values are loaded while a row is gathered.
         float val[6];
         float lo = read_lane_f(rowLo, r);
@@ -1958,19 +1949,14 @@ struct ColVisit {
                 eff[k] = win[k] & (unsigned)__builtin_amdgcn_sbfe((int)win[k], r + 16, 1);
             const float Df = I0f + lo;
             const int di = (int)lo;
-            if (cnt >= 3) pixels(Df, di, val, Three{});
-            else if (cnt == 2) pixels(Df, di, val, Two{});
-            else if (cnt == 1) pixels(Df, di, val, One{});
-            if (cnt >= 6) pixels(Df + 3.f, di + 3, val + 3, Three{});
-            else if (cnt == 5) pixels(Df + 3.f, di + 3, val + 3, Two{});
-            else if (cnt == 4) pixels(Df + 3.f, di + 3, val + 3, One{});
-            if (cnt > 6) {
-                for (int e = 6; e < cnt; e += 2) {  // one past the row's end weighs 0
-                    float xv[6];
-                    load(off + e, r, di + e, xv);
-                    pixels(Df + (float)e, di + e, xv, Two{});
-                }
-            }
+            col_row(cnt, [&](auto first, auto np) {
+                constexpr int F = decltype(first)::value;
+                pixels(F ? Df + (float)F : Df, di + F, val + F, np);
+            }, [&](int e, auto np) {
+                float xv[6];
+                load(off + e, r, di + e, xv);
+                pixels(Df + (float)e, di + e, xv, np);
+            });
             if (++r >= rEnd) break;
             lo = loN; cnt = cntN; off = offN;
             djf += 1.f;
@@ -2078,14 +2064,15 @@ __global__ __launch_bounds__(64 * BCW, MODE == COL_BACK ? 4 : 3) void col_kernel
 #define MGG_VISIT(KS) ColVisit<A, KS, MODE>::run(st, sacc[wv], im, M, cv, p.b.maskD2, ln, da, \
                                                        db, dzMax, oc, depth, D, p.b.hw, half, ua, ub, uc, va, vb, \
                                                        vc, na, nb, nc)
+            const int slots = __builtin_amdgcn_readfirstlane(col_slots(MODE, len));
             if constexpr (GATE) {
-                if (__builtin_amdgcn_readfirstlane(len < 5.f)) MGG_VISIT(5);
-                else if (__builtin_amdgcn_readfirstlane(len < 6.f)) MGG_VISIT(6);
+                if (slots == 5) MGG_VISIT(5);
+                else if (slots == 6) MGG_VISIT(6);
                 else MGG_VISIT(7);
             } else {
-                if (__builtin_amdgcn_readfirstlane(len < 6.f)) MGG_VISIT(6);
-                else if (__builtin_amdgcn_readfirstlane(len < 8.f)) MGG_VISIT(8);
-                else if (__builtin_amdgcn_readfirstlane(len < 10.f)) MGG_VISIT(10);
+                if (slots == 6) MGG_VISIT(6);
+                else if (slots == 8) MGG_VISIT(8);
+                else if (slots == 10) MGG_VISIT(10);
                 else MGG_VISIT(14);
             }
 #undef MGG_VISIT
