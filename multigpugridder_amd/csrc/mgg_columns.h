@@ -29,6 +29,9 @@ MGG_HD int col_slots(int mode, float len)
     return len < 6.f ? 6 : len < 8.f ? 8 : len < 10.f ? 10 : 14;
 }
 MGG_HD constexpr bool col_clamps(int mode, int slots) { return mode == COL_BACK ? slots == 7 : slots > 10; }
+// The same for slots looked up one by one (lanes at a half-integer index): of
+// an even number the last lies 125 entries below the last pair's.
+MGG_HD constexpr bool col_clamps_single(int mode, int slots) { return slots % 2 == 0 || col_clamps(mode, slots); }
 
 // A pixel offset is listed while its distance from the column along a cross
 // axis (frame components u, v) is at most this.

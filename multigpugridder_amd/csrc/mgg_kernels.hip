@@ -1887,7 +1887,7 @@ struct ColVisit {
             }
         };
         // only the longest columns reach past the table's ends
-        auto clampC = [](int i) { return col_clamps(MODE, K) ? min(max(i, ct_lo(MODE)), ct_hi(MODE) - 1) : i; };
+        auto clampTo = [](bool on, int i) { return on ? min(max(i, ct_lo(MODE)), ct_hi(MODE) - 1) : i; };
         float Ba, Bb, Bc;
         unsigned eff[GATE ? K : 1];
         // NP pixels of the current row from offset di on (bit di + 8 of eff).
@@ -1907,14 +1907,15 @@ struct ColVisit {
                 const int ic = cvt_rpi(sc[q]);
                 wab[q] = ct_pair<MODE>(st, cvt_rpi(fmaf(pa, SC, cA))).x * ct_pair<MODE>(st, cvt_rpi(fmaf(pb, SC, cB))).x;
 #pragma unroll
-                for (int h = 0; h < (K + 1) / 2; h++) wc[q][h] = ct_pair<MODE>(st, clampC(ic - 250 * h));
+                for (int h = 0; h < (K + 1) / 2; h++) wc[q][h] = ct_pair<MODE>(st, clampTo(col_clamps(MODE, K), ic - 250 * h));
             }
             if (__any(tie)) {
 #pragma unroll
                 for (int q = 0; q < NP; q++)
 #pragma unroll
                     for (int k = 0; k < K; k++) {
-                        float w = ct_pair<MODE>(st, clampC(cvt_rpi(fmaf(pc[q], SC, cC - 125.0f * k)))).x;
+                        const int i = cvt_rpi(fmaf(pc[q], SC, cC - 125.0f * k));
+                        float w = ct_pair<MODE>(st, clampTo(col_clamps_single(MODE, K), i)).x;
                         // keeps these loads apart from the paired ones (the
                         // compiler merges both into K single loads)
                         __asm__ volatile("" : "+v"(w));

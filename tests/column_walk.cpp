@@ -27,6 +27,15 @@ static std::vector<int> walk(int cnt)
 struct Angles { double th, ph, ps; };
 struct Reach { int slots; double lo, hi; };
 
+// How far the last index of a column lies below its first: slots are looked up
+// in pairs, and one by one.
+static double below(int mode, int slots)
+{
+    const int pairs = col_clamps(mode, slots) ? 0 : 250 * ((slots + 1) / 2 - 1);
+    const int singles = col_clamps_single(mode, slots) ? 0 : 125 * (slots - 1);
+    return pairs > singles ? pairs : singles;
+}
+
 // One frame's slots and its extreme indices, over all places where the column
 // can meet the plane (its remainder to the pixel grid and to the voxels).
 static Reach reach(int mode, const Angles &p, const std::vector<int> (&walks)[17])
@@ -70,7 +79,7 @@ static Reach reach(int mode, const Angles &p, const std::vector<int> (&walks)[17
     // (plus 5e-3 for rounding); the transpose counts the other way
     const double f = 0.5 * (std::fabs(u[c]) + std::fabs(v[c]));
     if (mode == COL_ADJOINT) { const double t = dlo; dlo = -dhi; dhi = -t; }
-    return {slots, 250.0 + 125.0 * (dlo - f + half + 5e-3 - 1.0) - 0.5 - 250.0 * ((slots + 1) / 2 - 1),
+    return {slots, 250.0 + 125.0 * (dlo - f + half + 5e-3 - 1.0) - 0.5 - below(mode, slots),
             250.0 + 125.0 * (dhi + f + half + 5e-3) + 0.5};
 }
 
@@ -95,7 +104,7 @@ int main(int argc, char **argv)
         for (int t = 0; t < 400000; t++) {
             const Angles p{std::acos(2.0 * uni(gen) - 1.0), 2.0 * M_PI * uni(gen), 2.0 * M_PI * uni(gen)};
             const Reach r = reach(mode, p, walks);
-            if (col_clamps(mode, r.slots)) continue;
+            if (col_clamps(mode, r.slots) && col_clamps_single(mode, r.slots)) continue;
             for (int sign : {-1, 1}) {
                 auto &list = best[{r.slots, sign}];
                 list.resize(8);
