@@ -405,6 +405,11 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
     const long long V3 = (long long)V * V * V;
     const T *vol = (const T *)p.vol;
 
+    // A tile with a pixel that a non-finite or huge direction sends where no
+    // box can follow takes neither the phase table nor a box: its taps are
+    // looked up one by one (entry 0 or 500) and gathered by checked loads.
+    const bool wild = __ballot(active && !(fabsf(x) + fabsf(y) + fabsf(z) < 4194304.0f)) != 0ull;
+
     float wi[NW], wj[NW], wk[NW];
     bool single = true;
     if constexpr (W4) {
@@ -423,8 +428,8 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
             const float sz = fmaf((float)(Zs + 3) - z, 125.0f, 250.0f);
             const bool odd = __builtin_amdgcn_fractf(sx) == 0.5f || __builtin_amdgcn_fractf(sy) == 0.5f ||
                              __builtin_amdgcn_fractf(sz) == 0.5f || !(fminf(x, fminf(y, z)) >= 1.0f);
-            single = __ballot(active && odd) != 0ull;
-            // (clamped: a non-finite coordinate stays inside the table)
+            single = wild || __ballot(active && odd) != 0ull;
+            // (clamped: any coordinate stays inside the table)
             const f4 qx = phase[min(max(cvt_rpi(sx) - 375, 0), 125)];
             const f4 qy = phase[min(max(cvt_rpi(sy) - 375, 0), 125)];
             const f4 qz = phase[min(max(cvt_rpi(sz) - 375, 0), 125)];
@@ -718,8 +723,8 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
     // The whole 8x8 tile; if its box is too large, its two 8x4 halves one
     // after the other; a half that still does not fit gathers from global
     // memory.
-    bool done = stageAndGather(0, FPT - 1, true, std::false_type{});
-    if (!done) {
+    bool done = !wild && stageAndGather(0, FPT - 1, true, std::false_type{});
+    if (!done && !wild) {
         const bool top = (ln >> 3) < FPT / 2;
         const bool d0 = stageAndGather(0, FPT / 2 - 1, top, std::true_type{});
         const bool d1 = stageAndGather(FPT / 2, FPT - 1, !top, std::true_type{});
