@@ -405,13 +405,9 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
     const long long V3 = (long long)V * V * V;
     const T *vol = (const T *)p.vol;
 
-    // A tile with a pixel that a non-finite or huge direction sends where no
-    // box can follow takes neither the phase table nor a box: its taps are
-    // looked up one by one (entry 0 or 500) and gathered by checked loads.
-    const bool wild = __ballot(active && !(fabsf(x) + fabsf(y) + fabsf(z) < 4194304.0f)) != 0ull;
-
     float wi[NW], wj[NW], wk[NW];
     bool single = true;
+    int least = NW;  // of a box's edges
     if constexpr (W4) {
         // The four entries of an axis' window lie 125 apart: one index, of the
         // last tap, and one row (T[k], T[k + 125], T[k + 250], T[k + 375]) of
@@ -426,13 +422,17 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
             const float sx = fmaf((float)(Xs + 3) - x, 125.0f, 250.0f);
             const float sy = fmaf((float)(Ys + 3) - y, 125.0f, 250.0f);
             const float sz = fmaf((float)(Zs + 3) - z, 125.0f, 250.0f);
-            const bool odd = __builtin_amdgcn_fractf(sx) == 0.5f || __builtin_amdgcn_fractf(sy) == 0.5f ||
-                             __builtin_amdgcn_fractf(sz) == 0.5f || !(fminf(x, fminf(y, z)) >= 1.0f);
-            single = wild || __ballot(active && odd) != 0ull;
-            // (clamped: any coordinate stays inside the table)
-            const f4 qx = phase[min(max(cvt_rpi(sx) - 375, 0), 125)];
-            const f4 qy = phase[min(max(cvt_rpi(sy) - 375, 0), 125)];
-            const f4 qz = phase[min(max(cvt_rpi(sz) - 375, 0), 125)];
+            const auto half = [](float s) {  // or NaN
+                const float f = __builtin_amdgcn_fractf(s);
+                return !(f < 0.5f || f > 0.5f);
+            };
+            const bool odd = half(sx) || half(sy) || half(sz) || !(fminf(x, fminf(y, z)) >= 1.0f);
+            single = __ballot(active && odd) != 0ull;
+            // a coordinate of NaN or beyond all volumes gets the row of zeros,
+            // as its lookups tap by tap read entries 0 and 500
+            const f4 qx = phase[min(max(cvt_rpi(sx), 374), 500) - 374];
+            const f4 qy = phase[min(max(cvt_rpi(sy), 374), 500) - 374];
+            const f4 qz = phase[min(max(cvt_rpi(sz), 374), 500) - 374];
 #pragma unroll
             for (int t = 0; t < NW; t++) {
                 wi[t] = qx[t];
@@ -442,6 +442,9 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         }
     }
     if (single) {
+        // A direction with an infinite component has pixels at 0 times infinity
+        // whose windows lie outside the box that the corners give: no box then.
+        if (__ballot(active && !(x + y + z == x + y + z)) != 0ull) least = INT_MAX;
 #pragma unroll
         for (int t = 0; t < NW; t++) {
             if (FAST) {
@@ -482,7 +485,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // Volume addressing by 32-bit byte offsets: from the volume's base
         // (below 4 GB), or (BIG) from the box's first element, whose
         // linear-index span is below 64 V^2 elements.
-        if (!(Dx >= NW && Dy >= NW && Dz >= NW && Dx <= 64 && Dy <= 64 && Dz <= 64 &&
+        if (!(Dx >= least && Dy >= NW && Dz >= NW && Dx <= 64 && Dy <= 64 && Dz <= 64 &&
               (BIG ? 64LL * V * V : V3) * (long long)sizeof(T) < (1LL << 32)))
             return false;
         // 16-byte segments per box row; for the 5-wide windows enough that the
@@ -508,7 +511,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // the volume offset and one for the LDS pointer.  The lane -> task
         // divisions use the reciprocal: (q + 0.5) / P is at least 0.5 / P
         // away from an integer, far more than its error for q, P <= 1024.
-        const int VV = V * V, V3i = (int)V3;
+        const int VV = V * V;
         const int P = Dy * segs;
         const float rP = __builtin_amdgcn_rcpf((float)P), rSegs = __builtin_amdgcn_rcpf((float)segs);
         const int G = P <= 64 ? __builtin_amdgcn_readfirstlane((int)(64.5f * rP)) : 1;
@@ -518,7 +521,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // needs a check.  lin grows with ez, ey and the segment, so the range
         // is spanned by the first and last segment of the box.
         const long long linLo = (long long)bz0 * VV + (long long)by0 * V + bx0;
-        const long long linHi = (long long)(bz0 + Dz - 1) * VV + (long long)(by0 + Dy - 1) * V + bx0 + 4 * segs - 1;
+        const long long linHi = linLo + (long long)(Dz - 1) * VV + (long long)(Dy - 1) * V + 4 * segs - 1;
         const bool boxIn = linLo >= 0 && linHi < V3;
         // Four planes per batch (three with the 16-bit types' conversions): all
         // loads of a batch are in flight before the first LDS store waits on
@@ -529,9 +532,11 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // a 32-bit byte offset from the volume's base, or (BIG: volumes of
         // 4 GB and more) from the box's first element; the checked one, which
         // runs only on boxes that cross the volume's index range, by the
-        // int linear index, or (BIG) a 64-bit one.
+        // linear index in 32 or (BIG) 64 bits, unsigned: it wraps for boxes
+        // at infinity, and as a signed one could pass the test in 32 bits and
+        // be an address in 64.
         const T *volBox = vol + ((BIG && boxIn) ? linLo : 0);
-        using Lin = std::conditional_t<BIG, long long, int>;
+        using Lin = std::conditional_t<BIG, unsigned long long, unsigned>;
         constexpr int SB = DT == DT_F32 ? 4 : 3;
         const int lStep = G * VV, dStep = G * PP;
         for (int c = 0; c < nLanePass; c++) {
@@ -541,7 +546,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
             const int ey = (int)(((float)pq + 0.5f) * rSegs);
             const int sg = pq - ey * segs;
             if (pl >= G) continue;
-            const Lin lin0 = (Lin)(bz0 + pl) * VV + (Lin)(by0 + ey) * V + (bx0 + 4 * sg);
+            const Lin lin0 = ((Lin)bz0 + (Lin)pl) * (Lin)VV + ((Lin)by0 + (Lin)ey) * (Lin)V + ((Lin)bx0 + (Lin)(4 * sg));
             float *d0 = box + pl * PP + ey * RP + 4 * sg;
             auto stage = [&](auto inBox) {
                 // offset from volBox (BIG and boxIn: inside the box's span,
@@ -554,13 +559,15 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
 #pragma unroll
                     for (int k = 0; k < SB; k++) {
                         if (ez + k * G < Dz) {
-                            const Idx lk = l + (Idx)k * lStep;
+                            const Idx lk = l + (Idx)(k * lStep);
                             if (decltype(inBox)::value) {
                                 load4<L>((const T *)((const char *)volBox + (unsigned)lk * (unsigned)sizeof(T)), v4[k]);
                             } else {
 #pragma unroll
-                                for (int e = 0; e < 4; e++)
-                                    v4[k][e] = (lk + e >= 0 && lk + e < (BIG ? (Lin)V3 : (Lin)V3i)) ? L::one(vol + lk + e) : 0.f;
+                                for (int e = 0; e < 4; e++) {
+                                    const Lin le = (Lin)lk + (Lin)e;
+                                    v4[k][e] = le < (Lin)V3 ? L::one(vol + le) : 0.f;
+                                }
                             }
                         }
                     }
@@ -571,7 +578,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
                             *(f4 *)(dp + k * dStep) = w4;
                         }
                     }
-                    l += SB * lStep;
+                    l += (Idx)(SB * lStep);
                     dp += SB * dStep;
                 }
             };
@@ -723,8 +730,8 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
     // The whole 8x8 tile; if its box is too large, its two 8x4 halves one
     // after the other; a half that still does not fit gathers from global
     // memory.
-    bool done = !wild && stageAndGather(0, FPT - 1, true, std::false_type{});
-    if (!done && !wild) {
+    bool done = stageAndGather(0, FPT - 1, true, std::false_type{});
+    if (!done) {
         const bool top = (ln >> 3) < FPT / 2;
         const bool d0 = stageAndGather(0, FPT / 2 - 1, top, std::true_type{});
         const bool d1 = stageAndGather(FPT / 2, FPT - 1, !top, std::true_type{});
@@ -738,7 +745,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
             for (int bb = 0; bb < NW; bb++)
 #pragma unroll
                 for (int aa = 0; aa < NW; aa++) {
-                    const long long lin = (long long)(Zs + cc) * V * V + (long long)(Ys + bb) * V + (Xs + aa);
+                    const long long lin = ((long long)Zs + cc) * V * V + ((long long)Ys + bb) * V + ((long long)Xs + aa);
                     if (lin < V3 && lin >= 0) sc = fmaf(wi[aa] * wj[bb], L::one(vol + lin), sc);
                 }
             acc = fmaf(wk[cc], sc, acc);
@@ -778,14 +785,15 @@ __device__ __forceinline__ bool fp_win4(const unsigned *check)
     return check != nullptr && __builtin_amdgcn_readfirstlane(*check) == 1u;
 }
 
-// Rows (T[k], T[k + 125], T[k + 250], T[k + 375]), k <= 125, of the 501-entry
-// table, by the whole workgroup.
-constexpr int FPPHASE = 126;
+// A row of zeros, then (T[k], T[k + 125], T[k + 250], T[k + 375]), k <= 125, of
+// the 501-entry table, by the whole workgroup.
+constexpr int FPPHASE = 127;
 __device__ __forceinline__ void fp_phase_table(f4 *__restrict__ phase, const float *__restrict__ ker)
 {
     for (int k = threadIdx.x; k < FPPHASE; k += kThreads) {
-        const f4 row = {ker[k], ker[k + 125], ker[k + 250], ker[k + 375]};
-        phase[k] = row;
+        const float *t = ker + max(k - 1, 0);
+        const f4 row = {t[0], t[125], t[250], t[375]};
+        phase[k] = k > 0 ? row : f4{0.f, 0.f, 0.f, 0.f};
     }
     __syncthreads();
 }
