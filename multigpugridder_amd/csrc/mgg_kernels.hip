@@ -235,8 +235,9 @@ __global__ __launch_bounds__(kThreads) void fp_kernel(FPArgs p)
 #pragma unroll
                 for (int bb = 0; bb < 5; bb++) wij[aa][bb] = wi[aa] * wj[bb];
 
-            const bool fast = X >= 2 && X + 2 + L::kRowSlack < V && Y >= 2 && Y + 2 < V &&
-                              Z >= 2 && Z + 2 < V;
+            // unsigned: X may be INT_MAX (a non-finite direction)
+            const unsigned top = (unsigned)max(V - 4, 0), topX = (unsigned)max(V - 4 - L::kRowSlack, 0);
+            const bool fast = (unsigned)X - 2u < topX && (unsigned)Y - 2u < top && (unsigned)Z - 2u < top;
             if (fast) {
                 const T *base = vol + (((size_t)(Z - 2) * V + (size_t)(Y - 2)) * V + (X - 2));
 #pragma unroll
@@ -260,8 +261,8 @@ __global__ __launch_bounds__(kThreads) void fp_kernel(FPArgs p)
                     for (int bb = 0; bb < 5; bb++)
 #pragma unroll
                         for (int cc = 0; cc < 5; cc++) {
-                            long long lin = (long long)(Z - 2 + cc) * V * V +
-                                            (long long)(Y - 2 + bb) * V + (X - 2 + aa);
+                            long long lin = ((long long)Z - 2 + cc) * V * V +
+                                            ((long long)Y - 2 + bb) * V + ((long long)X - 2 + aa);
                             if (lin < V3 && lin >= 0)
                                 acc = fmaf(wij[aa][bb] * wk[cc], L::one(vol + lin), acc);
                         }
@@ -1302,8 +1303,8 @@ __global__ __launch_bounds__(kThreads) void bp_kernel(BPArgs p)
                         w = w * sker[kb_index(py - fvj, p.fW, p.kerScale, p.kerCenter, p.K)];
                         const float pz = fmaf(Di[ii], u2, Bz[jj]) + cvf;
                         w = w * sker[kb_index(pz - fvk, p.fW, p.kerScale, p.kerCenter, p.K)];
-                        const int lin = (J - 2 + jj) * M + (I - 2 + ii);
-                        if (lin >= 0 && lin < M2) {
+                        const unsigned lin = ((unsigned)J - 2u + jj) * (unsigned)M + ((unsigned)I - 2u + ii);
+                        if (lin < (unsigned)M2) {
                             cum = cum + im[lin] * w;
                             if (DENS) dsum = dsum + w;
                         }
@@ -1320,8 +1321,8 @@ __global__ __launch_bounds__(kThreads) void bp_kernel(BPArgs p)
                         w = w * sker[kb_index(py - fvj, p.fW, p.kerScale, p.kerCenter, p.K)];
                         const float pz = ref_sum2c(ti, u2, tj, v2, cvf);
                         w = w * sker[kb_index(pz - fvk, p.fW, p.kerScale, p.kerCenter, p.K)];
-                        const int lin = j1 * M + i1;
-                        if (lin >= 0 && lin < M2) {
+                        const unsigned lin = (unsigned)j1 * (unsigned)M + (unsigned)i1;
+                        if (lin < (unsigned)M2) {
                             cum = cum + im[lin] * w;
                             if (DENS) dsum = dsum + w;
                         }
@@ -1590,13 +1591,17 @@ __global__ __launch_bounds__(64 * BFW) void bp_fast_kernel(BPArgs p)
 #pragma unroll
                     for (int s5 = 0; s5 < 5; s5++) Di[s5] = (float)(I - 2 + s5 - ci);
                     float cum = 0.f, dsum = 0.f;
-                    const bool inside = I >= 2 && I + 2 < M && J >= 2 && J + 2 < M;
+                    // unsigned, as the linear index below: I and J may be INT_MAX (a
+                    // non-finite direction), where a signed sum could pass the test
+                    // wrapped and be an address unwrapped
+                    const unsigned top = (unsigned)max(M - 4, 0);
+                    const bool inside = (unsigned)I - 2u < top && (unsigned)J - 2u < top;
 #pragma unroll 1
                     for (int jj = 0; jj < 5; jj++) {
                         const float dj = (float)(J - 2 + jj - ci);
                         const float Bx = dj * v0, By = dj * v1, Bz = dj * v2;
                         float val[5], vin[5];  // image values; 1 where the tap is in bounds, else 0
-                        const int row = (J - 2 + jj) * M + (I - 2);
+                        const unsigned row = ((unsigned)J - 2u + jj) * (unsigned)M + ((unsigned)I - 2u);
                         if (inside) {
                             f4 a;
                             __builtin_memcpy(&a, im + row, 16);
@@ -1609,8 +1614,8 @@ __global__ __launch_bounds__(64 * BFW) void bp_fast_kernel(BPArgs p)
                             // (gpuBackProject.cu:99): wraps across rows.
 #pragma unroll
                             for (int ii = 0; ii < 5; ii++) {
-                                const int lin = row + ii;
-                                const bool ok = lin >= 0 && lin < M2;
+                                const unsigned lin = row + ii;
+                                const bool ok = lin < (unsigned)M2;
                                 val[ii] = ok ? im[lin] : 0.f;
                                 vin[ii] = ok ? 1.f : 0.f;
                             }
