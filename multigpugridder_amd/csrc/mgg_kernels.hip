@@ -301,12 +301,16 @@ __global__ __launch_bounds__(kThreads) void fp_kernel(FPArgs p)
 // accumulation rounding differs.
 // ---------------------------------------------------------------------------
 constexpr int FPT = 8;          // tile edge (pixels)
-// Per-wave staged box budget (floats).  Four boxes and the phase table take
-// 40,928 bytes of LDS, a quarter of the CU's 160 KB, so four workgroups share a
-// CU (the kernel's 125 VGPRs allow four waves per SIMD, at most 128 do); nearly
-// every 8x8 tile's box of the 4x4x4 windows fits whole, the rest are staged as
-// two 8x4 halves.  Five workgroups per CU with 1,920 floats ran 10% slower.
-constexpr int FPBOX = 2432;     // per-wave staged box budget (floats)
+// Per-wave staged box budgets (floats): 5-wide windows and the transpose, and
+// 4-wide windows, which leave room for the phase table.  Four boxes take at
+// most 40,960 bytes of LDS, a quarter of the CU's 160 KB, so four workgroups
+// share a CU (the kernel's VGPRs allow four waves per SIMD).  The median box
+// of an 8x8 tile's 5-wide windows at N=128 holds 2,464 floats; nearly every
+// box of the 4-wide ones fits.  Boxes that do not are staged as two 8x4
+// halves.  Five workgroups per CU with 1,920 floats ran the 4-wide gather 10%
+// slower.
+constexpr int FPBOX = 2560;
+constexpr int FPBOX4 = 2432;
 constexpr int FPKER = 640;      // generic-table path: table floats kept in LDS
 
 __device__ __forceinline__ void wave_lds_sync_fp()
@@ -377,7 +381,7 @@ __device__ __forceinline__ void load4<VolLoad<DT_F16>>(const uint16_t *p, float 
 // gives the same sums bit for bit, and the box shrinks to the voxels the
 // windows touch: [floor(min) - 1, floor(max) + 2] per axis instead of
 // [floor(min) - 2, ceil(max) + 2], about 40% fewer voxels to stage.
-template <int DT, bool FAST, bool W4, bool BIG>
+template <int DT, bool FAST, bool W4, bool BIG, int BOX>
 __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *__restrict__ sker,
                                                  const f4 *__restrict__ phase, float *__restrict__ box, int a, int i0,
                                                  int j0, int ln, bool active, bool pix, float *out)
@@ -499,11 +503,11 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // bank offset); otherwise the rows are packed.
         int RP = (segs | 1) * 4;
         int PP = RP * Dy + ((Dy & 1) ? 0 : RP);
-        if (PP * Dz > FPBOX) {
+        if (PP * Dz > BOX) {
             RP = segs * 4;
             PP = RP * Dy;
         }
-        if (PP * Dz > FPBOX) return false;
+        if (PP * Dz > BOX) return false;
 
         // Stage.  A plane of the box holds P = Dy * segs row segments.  With
         // P <= 64 one pass covers G = 64 / P planes (lane -> plane offset pl,
@@ -524,11 +528,12 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         const long long linLo = (long long)bz0 * VV + (long long)by0 * V + bx0;
         const long long linHi = linLo + (long long)(Dz - 1) * VV + (long long)(Dy - 1) * V + 4 * segs - 1;
         const bool boxIn = linLo >= 0 && linHi < V3;
-        // Four planes per batch (three with the 16-bit types' conversions): all
-        // loads of a batch are in flight before the first LDS store waits on
-        // them (2, 3, 4, 5 and 6 planes: 2.17, 2.10, 2.07, 2.08 and 2.08 ms per
-        // 2,000 directions at N=128; BF16, 500 at N=256: 2.49, 2.28, -, 2.45
-        // and 2.48 ms; 8 needs more than 128 VGPRs, three waves per SIMD).  The checked and unchecked variants are separate loops
+        // Four planes per batch (three with the 16-bit types' conversions; six
+        // for 5-wide windows): all loads of a batch are in flight before the
+        // first LDS store waits on them (2, 3, 4, 5 and 6 planes: 2.17, 2.10,
+        // 2.07, 2.08 and 2.08 ms per 2,000 directions at N=128; BF16, 500 at
+        // N=256: 2.49, 2.28, -, 2.45 and 2.48 ms; 8 needs more than 128 VGPRs,
+        // three waves per SIMD).  The checked and unchecked variants are separate loops
         // (boxIn is wave-uniform).  The unchecked one addresses the volume by
         // a 32-bit byte offset from the volume's base, or (BIG: volumes of
         // 4 GB and more) from the box's first element; the checked one, which
@@ -538,7 +543,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
         // be an address in 64.
         const T *volBox = vol + ((BIG && boxIn) ? linLo : 0);
         using Lin = std::conditional_t<BIG, unsigned long long, unsigned>;
-        constexpr int SB = DT == DT_F32 ? 4 : 3;
+        constexpr int SB = DT != DT_F32 ? 3 : W4 ? 4 : 6;
         const int lStep = G * VV, dStep = G * PP;
         for (int c = 0; c < nLanePass; c++) {
             const int q = ln + 64 * c;
@@ -757,7 +762,7 @@ __device__ __forceinline__ void fp_lds_tile_body(const FPArgs &p, const float *_
 
 // One 8x8 tile of one direction; W4 (only with the 501-entry table) selects
 // the 4-wide windows.
-template <int DT, bool FAST, bool W4, bool BIG = false>
+template <int DT, bool FAST, bool W4, bool BIG, int BOX>
 __device__ __forceinline__ void fp_lds_tile(const FPArgs &p, const float *__restrict__ sker,
                                             const f4 *__restrict__ phase, float *__restrict__ box, int a, int tx, int ty,
                                             int ln)
@@ -775,7 +780,7 @@ __device__ __forceinline__ void fp_lds_tile(const FPArgs &p, const float *__rest
         if (pix) *out = 0.f;
         return;
     }
-    fp_lds_tile_body<DT, FAST, FAST && W4, BIG>(p, sker, phase, box, a, i0, j0, ln, active, pix, out);
+    fp_lds_tile_body<DT, FAST, FAST && W4, BIG, BOX>(p, sker, phase, box, a, i0, j0, ln, active, pix, out);
 }
 
 // The 4-wide windows need a finite volume and a finite 501-entry table whose
@@ -803,8 +808,10 @@ template <int DT, bool FAST, bool BIG>
 __global__ __launch_bounds__(kThreads) void fp_lds_kernel(FPArgs p)
 {
     __shared__ float sker[FPKER];
-    __shared__ __attribute__((aligned(16))) float sbox[4][FPBOX];
-    __shared__ f4 sphase[FAST ? FPPHASE : 1];
+    // four boxes of 5-wide windows, or four boxes of 4-wide ones and the phase table
+    __shared__ __attribute__((aligned(16))) float sbox[4 * FPBOX];
+    static_assert(4 * FPPHASE + 4 * FPBOX4 <= 4 * FPBOX, "the phase table and its boxes");
+    f4 *const sphase = (f4 *)(sbox + 4 * FPBOX4);
 
     if (!FAST) {  // the fast lookup reads the table from global memory
         for (int t = threadIdx.x; t < p.K; t += kThreads) sker[t] = p.ker[t];
@@ -821,8 +828,10 @@ __global__ __launch_bounds__(kThreads) void fp_lds_kernel(FPArgs p)
             const unsigned r = wk.cols(t), row = band * wk.bandRows + r, col = t - r * wk.cols.d;
             const int tx = (int)(2u * col) + (wv & 1), ty = (int)(2u * row) + (wv >> 1);
             if (unit >= wk.units || row >= wk.rows || tx >= p.tilesPerRow || ty >= p.tilesPerRow) continue;
-            fp_lds_tile<DT, FAST, decltype(win4)::value, BIG>(p, sker, decltype(win4)::value ? sphase : nullptr, sbox[wv],
-                                                              (int)a, tx, ty, ln);
+            constexpr bool W4 = decltype(win4)::value;
+            constexpr int BOX = W4 ? FPBOX4 : FPBOX;
+            fp_lds_tile<DT, FAST, W4, BIG, BOX>(p, sker, W4 ? sphase : nullptr, sbox + wv * BOX,
+                                                (int)a, tx, ty, ln);
         }
     };
     // The window width is chosen once, outside the tile loop, so that each
@@ -897,7 +906,7 @@ __global__ __launch_bounds__(kThreads) void adj_kernel(FPArgs p, const float *__
 template <int DT, bool BIG>
 __global__ __launch_bounds__(kThreads) void fp_lds_multi_kernel(FPMultiArgs m)
 {
-    __shared__ __attribute__((aligned(16))) float sbox[4][FPBOX];
+    __shared__ __attribute__((aligned(16))) float sbox[4][FPBOX4];
     __shared__ f4 sphase[FPPHASE];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
     fp_phase_table(sphase, m.seg[0].ker);  // segments with another table look up tap by tap
@@ -919,8 +928,8 @@ __global__ __launch_bounds__(kThreads) void fp_lds_multi_kernel(FPMultiArgs m)
         const unsigned local = work - sg.workStart;
         const int d = (int)(local / (unsigned)sg.tilesPerImg), tile = (int)(local - (unsigned)d * (unsigned)sg.tilesPerImg);
         const int ty = tile / sg.tilesPerRow, tx = tile - ty * sg.tilesPerRow;
-        if (fp_win4(sg.check)) fp_lds_tile<DT, true, true, BIG>(a, nullptr, phase, sbox[wv], d, tx, ty, ln);
-        else fp_lds_tile<DT, true, false, BIG>(a, nullptr, nullptr, sbox[wv], d, tx, ty, ln);
+        if (fp_win4(sg.check)) fp_lds_tile<DT, true, true, BIG, FPBOX4>(a, nullptr, phase, sbox[wv], d, tx, ty, ln);
+        else fp_lds_tile<DT, true, false, BIG, FPBOX4>(a, nullptr, nullptr, sbox[wv], d, tx, ty, ln);
     }
 }
 
