@@ -167,6 +167,7 @@ struct FPWalk {
     FastDiv bands;      // units per image
     unsigned rows, bandRows;  // workgroup tile rows of an image, of a band
     unsigned units, perXcd;   // units in all; workgroup tiles of one XCD's list
+    unsigned turn;            // 7: the XCDs change places from 8 units to the next (bands), 0: not
 };
 
 struct FPArgs {
@@ -823,7 +824,7 @@ __global__ __launch_bounds__(kThreads) void fp_lds_kernel(FPArgs p)
     auto walk = [&](auto win4) {
         for (unsigned it = blockIdx.x >> 3; it < wk.perXcd; it += gridDim.x >> 3) {
             const unsigned k = wk.unitTiles(it), t = it - k * wk.unitTiles.d;
-            const unsigned unit = xcd + 8u * k;
+            const unsigned unit = ((xcd + (k & wk.turn)) & 7u) + 8u * k;
             const unsigned a = wk.bands(unit), band = unit - a * wk.bands.d;
             const unsigned r = wk.cols(t), row = band * wk.bandRows + r, col = t - r * wk.cols.d;
             const int tx = (int)(2u * col) + (wv & 1), ty = (int)(2u * row) + (wv >> 1);
@@ -4021,12 +4022,13 @@ hipError_t launch_forward_project(const void *vol, int dtype, const ProjGeom &g,
         if (work > 0xffffffffull / 2) return hipErrorInvalidValue;
         a.totalWork = (unsigned)work;
         a.perXcd = 0;
-        // Units of whole images from 64 directions on; bands below, so that every
-        // XCD has work.
+        // Units of whole images from 256 directions on, where the XCDs' shares
+        // even out; bands below (64 directions at N=256: 328 us against 337 by
+        // whole images, 5-wide windows 502 against 529).
         FPWalk &wk = a.walk;
         const unsigned cols = (unsigned)(a.tilesPerRow + 1) / 2;
         unsigned bands = 1;
-        while (bands < 8 && bands < cols && (unsigned)nAxes * bands < 64u) bands *= 2;
+        while (bands < 8 && bands < cols && (unsigned)nAxes * bands < 256u) bands *= 2;
         wk.rows = cols;
         wk.bandRows = (cols + bands - 1) / bands;
         wk.cols.set(cols);
@@ -4034,10 +4036,26 @@ hipError_t launch_forward_project(const void *vol, int dtype, const ProjGeom &g,
         wk.unitTiles.set(cols * wk.bandRows);
         wk.units = (unsigned)nAxes * bands;
         wk.perXcd = (wk.units + 7) / 8 * cols * wk.bandRows;
-        // Four tiles per wave, a stride of the grid apart: 2,000 random
-        // directions at N=128 in 2.32 / 2.12 / 2.06 / 2.07 / 2.09 ms with 1 /
-        // 2 / 3 / 4 / 6, 16 in 27 / 27 / 35 / 27 / 30 us.
-        const unsigned tpw = 4;
+        // A band meets the mask's disc more or less by its place in the image,
+        // so each XCD takes every place in turn (16 directions at N=256: 88 ->
+        // 85 us, 5-wide windows 146 -> 137).
+        wk.turn = bands > 1 ? 7u : 0u;
+        // Tiles per wave, a stride of the grid apart: the most that do not
+        // leave the last round of the card's 1,024 resident workgroups short,
+        // by the cost of 1 / 2 / 3 / 4 of them in a long launch (2,000 random
+        // directions at N=128: 2.33 / 2.13 / 2.07 / 2.07 ms; without a check,
+        // and so a phase table, 64 at N=256: 530 / 531 / 542 / 548 us).  16
+        // directions at N=96, 2,304 workgroup tiles: 17.3 / 19.4 / 16.8 / 19.6
+        // us; 2 at N=64, unchecked: 11.5 / 13.5 / 19.4 / 24.8 us.
+        const double checked[5] = {0.0, 1.12, 1.03, 1.0, 1.0}, unchecked[5] = {0.0, 1.03, 1.0, 1.02, 1.02};
+        const double *weight = a.check ? checked : unchecked;
+        const double tiles = 8.0 * wk.perXcd;
+        unsigned tpw = 4;
+        double least = 0.0;
+        for (unsigned k = 4; k >= 1; k--) {
+            const double cost = std::ceil(tiles / (1024.0 * k)) * k * weight[k];
+            if (k == 4 || cost < least) least = cost, tpw = k;
+        }
         const dim3 grid((wk.perXcd + tpw - 1) / tpw * 8), block(kThreads);
         // volumes of 4 GB and more: box addressing from the box's first element
         const int esz = dtype == DT_F32 ? 4 : 2;
