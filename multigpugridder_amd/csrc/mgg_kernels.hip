@@ -2626,7 +2626,7 @@ __global__ __launch_bounds__(256) void k_inv_rows(const float *__restrict__ cas,
         const float *rowB = cas + (size_t)a * M * M + (size_t)mirror_idx<M>(ky) * M;
         // Unconditional loads (every address is inside the image), so that all
         // 2R are in flight before the first use; the CAS index 0 row and column
-        // and rows beyond M/2 select zero afterwards.
+        // select zero afterwards (rows beyond M/2 are not stored).
         float c1[R], c2[R];
 #pragma unroll
         for (int n2 = 0; n2 < R; n2++) {
@@ -2638,8 +2638,13 @@ __global__ __launch_bounds__(256) void k_inv_rows(const float *__restrict__ cas,
 #pragma unroll
         for (int n2 = 0; n2 < R; n2++) {
             const int kx = t + 16 * n2;
-            const float sg = (rowOk && kx != 0 && ky != 0) ? chk(kx + ky) : 0.f;
+            const float sg = chk(kx + ky);
             v[n2] = make_float2(sg * (0.5f * (c1[n2] + c2[n2])), sg * (0.5f * (c1[n2] - c2[n2])));
+        }
+        if (t == 0) v[0] = make_float2(0.f, 0.f);  // kx = 0, NaN included
+        if (ky == 0) {
+#pragma unroll
+            for (int n2 = 0; n2 < R; n2++) v[n2] = make_float2(0.f, 0.f);
         }
         __syncthreads();
         fft_m<R, 1>(v, t, ex, tw);
