@@ -71,6 +71,13 @@ def _n_axes(axes: torch.Tensor) -> int:
     return axes.numel() // 9
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two contiguous tensors share memory, by address: tensors of
+    different storages can."""
+    a0, b0 = a.data_ptr(), b.data_ptr()
+    return a0 < b0 + b.numel() * b.element_size() and b0 < a0 + a.numel() * a.element_size()
+
+
 def _same_device(*named):
     devs = {(n, t.device) for n, t in named if t is not None}
     if len({d for _, d in devs}) > 1:
@@ -267,11 +274,9 @@ def cas_images_to_images(cas_images: torch.Tensor, n: int, out: torch.Tensor | N
         _need_numel(out, p * n * n, "out")
     _same_device(("cas_images", cas_images), ("out", out))
     _check(cas_images, "cas_images")
+    shared = out is not None and _overlap(cas_images, out)
     if out is None:
         out = torch.empty((p, n, n), device=cas_images.device, dtype=torch.float32)
-        shared = False
-    else:
-        shared = out.untyped_storage().data_ptr() == cas_images.untyped_storage().data_ptr()
     src = cas_images if clobber or (not shared and _lib.image_chain_reads_only(m, n)) else cas_images.clone()
     _check(out, "out")
     _lib.call("mgg_op_cas_images_to_images", _ptr(src), _ptr(out), p, m, n, _stream())
