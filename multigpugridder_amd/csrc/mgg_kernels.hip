@@ -4244,19 +4244,38 @@ hipError_t launch_back_project_adjoint(float *volAcc, const ProjGeom &g, const f
     return hipGetLastError();
 }
 
-// Where the column kernels win (they cost more per block, bp_fast_kernel and
-// the tiles' atomics more per direction), ms by columns / by the other kernel,
-// random directions:
-//   back projection  N=64: 500 0.7/1.38 (100: 0.25/0.16); N=96: 256 0.66/0.76, 1,000 2.05/3.01;
-//     N=128: 256 1.10/0.89, 800 2.74/2.70, 1,500 4.80/5.13; N=192: 300 2.84/2.77, 600 4.77/5.21;
-//     N=256: 300 5.53/5.55
-//   transpose  N=64: 1,500 2.64/2.17; N=96: 256 0.93/0.81, 1,000 2.92/3.13; N=128: 256 1.48/1.60,
-//     800 3.77/5.00; N=192: 100 1.82/1.24, 600 6.33/7.33; N=256: 300 6.82/6.67
+// Distance of the volume's centre from the nearest face of the bricks of 8: 0
+// (the centre is on a face, or the voxel before one), 1, or 2 and more.  With the
+// centre well inside a brick that brick meets every direction and sets the
+// time; on a corner eight share them (4 waves, 1,000 directions: N=92 1.90 ms,
+// N=96 2.94).
+static int centre_depth(int V)
+{
+    const int c = V / 2 % 8;
+    return std::min(c, 7 - c);
+}
+
+// Where the column kernels win (they cost more per block, the bricks by their
+// central one, the tiles' atomics more per direction).  Time by columns over
+// the time by the better number of waves per brick, random directions:
+//   centre depth 0  N=60: 256 1.42, 500 1.21, 1,000 1.06; N=76: 1.33, 1.14, 0.96; N=92: 1.28, 1.11, 0.98;
+//     N=100: 1.45, 1.27, 1.11, 1,500 1.04; N=116: 1.30, 1.16, 1.03, 1.00; N=124: 1.28, 1.15, 1.02, 0.99
+//   1  N=62: 256 1.30, 500 1.11, 1,000 0.94; N=86: 1.10, 1.06, 0.93; N=102: 1.25, 1.07, 0.92; N=110: 1.33, 1.20, 1.04
+//   2, 3  N=32: 256 0.59; N=64: 256 1.12, 500 0.94; N=80: 500 1.04, 1,000 0.87; N=88: 256 1.04, 500 1.00; N=96: 256 0.93;
+//     N=104: 256 1.04, 500 0.91; N=112: 256 1.11, 500 0.99; N=120: 500 1.13, 1,000 0.97; N=128: 1,000 0.98
+//   N=140: 700 1.00, 1,000 0.96; N=160: 500 1.03; N=192: 500 0.98; N=256: 500 0.94
+// The transpose over the tiles: N=80 1,000 0.99; N=96: 500 1.02, 700 0.94; N=108: 500 0.95; N=112: 256 1.05, 500 0.96;
+//   N=120: 256 1.04, 500 0.94; N=124: 256 1.00; N=128: 256 0.91; N=146: 256 1.00; N=160: 350 0.98, 500 0.91
 bool uses_columns(const ProjGeom &g, int nAxes, ColKind kind)
 {
     const bool adjoint = kind == ColKind::Adjoint;
-    const int least = adjoint ? (g.V < 190 ? INT_MAX : g.V < 230 ? 800 : g.V < 300 ? 256 : 500)
-                              : (g.V < 230 ? 256 : g.V < 300 ? 1000 : 500);
+    const int depth = centre_depth(g.V);
+    const int least = adjoint ? (g.V < 190 ? INT_MAX : g.V < 230 ? 800 : g.V < 250 ? 500 : g.V < 300 ? 256 : 500)
+                      : g.V >= 300 ? 500
+                      : g.V >= 240 ? 1000
+                      : depth == 0 ? 1500
+                      : depth == 1 ? 800
+                      : g.V < 110 || (g.V >= 180 && g.V < 220) ? 256 : 500;
     if (nAxes < least || !bp_uses_fast_path(g)) return false;
     const BPArgs a = bp_args(nullptr, nullptr, g, nullptr, nAxes, nullptr);
     if (a.maskD2 < 0) return false;
@@ -4268,14 +4287,17 @@ bool uses_columns(const ProjGeom &g, int nAxes, ColKind kind)
 }
 
 // Waves per brick of bp_fast_kernel.  A small volume's bricks do not fill the
-// GPU, and the central ones, which every direction crosses, set the time:
-// eight waves halve it (N=64, 100 directions: 0.28 -> 0.16 ms; with the
-// density, 777: 2.26 -> 1.25 ms; N=96, 512: 1.53 -> 1.41 ms); elsewhere the
-// passes' leftover groups of more waves cost more (N=96, 64 directions: 0.19
-// -> 0.26 ms; N=128, 2,000: 6.9 -> 10.6 ms).
+// GPU, and the central ones set the time: eight waves halve it (the density the
+// same).  Elsewhere the passes' leftover groups of more waves cost more.  Time
+// with eight waves over four: N=38 1 direction 0.98, 8 0.75; N=48 1 1.08, 16
+// 0.70; N=64 16 1.21, 32 0.80; N=68 32 1.14, 64 0.85; N=72 32 1.09, 64 0.74;
+// N=77 64 1.09, 128 0.90; N=80 128 0.68; N=84 128 1.09 (centre depth 0), N=88
+// 0.84, N=90 0.96 (2, 3); N=100 256 1.50; N=104 256 1.15.
 static int bp_fast_waves(int V, int nAxes)
 {
-    return V <= 80 || (V <= 160 && nAxes >= 32) || (V <= 210 && nAxes >= 256) ? 8 : 4;
+    const int least = V <= 82 ? 0 : V <= 110 ? 16 : V <= 140 ? 32 : V <= 150 ? 64
+                      : V <= 172 || (V <= 190 && centre_depth(V) >= 2) ? 128 : INT_MAX;
+    return nAxes >= least ? 8 : 4;
 }
 
 int col_depth(ColKind kind) { return bc_depth((int)kind); }
@@ -4322,10 +4344,10 @@ hipError_t launch_columns(ColKind kind, float *volAcc, const ProjGeom &g, const 
         a.reachD2 = (int)std::ceil(r * r);
     }
     // Small volumes have few blocks, and the central ones' chain of directions
-    // sets the time: eight waves share it (N=64, 777 directions: 1.41 -> 1.00
-    // ms; N=96: 1.14 -> 1.31, N=128: 6.46 -> 6.80 for 2,000).
+    // sets the time: eight waves share it (time over four waves': N=64, 500
+    // directions 0.68; N=80 0.87; N=84 0.94; N=92 1.11; N=96, 256 1.20).
     if (kind == ColKind::Adjoint) col_launches<COL_ADJOINT, 4>(a, (unsigned)orderLen, s);
-    else if (g.V <= 160) col_launches<COL_BACK, 8>(a, (unsigned)orderLen, s);
+    else if (g.V <= 176) col_launches<COL_BACK, 8>(a, (unsigned)orderLen, s);
     else col_launches<COL_BACK, 4>(a, (unsigned)orderLen, s);
     return hipGetLastError();
 }
