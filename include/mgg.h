@@ -230,9 +230,9 @@ int mgg_op_cas_images_to_images(float *cas_images, float *images, int n, int m, 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): mgg_op_cas_images_to_images without any allocation and
- * without clobbering cas_images.  Only the fused chains' sizes are accepted
- * (m = 128, 192, 256, 384 or 512, nn <= m, m - nn even; others return
- * MGG_ERR_UNSUPPORTED); the intermediate lives in a fixed 32 MiB device array
+ * without clobbering cas_images.  Only m = 128, 192, 256, 384 and 512 are
+ * accepted (nn <= m, m - nn even; others return MGG_ERR_UNSUPPORTED, also
+ * those whose chain needs no plan); the intermediate lives in a fixed 32 MiB device array
  * per GPU, held from library load to process end, and n is processed in chunks
  * that fit it.  Calls that overlap on one GPU share that array and race:
  * order them on one stream. */

@@ -897,8 +897,7 @@ int mgg_op_cas_images_to_images_noalloc(const float *cas_images, float *images, 
             raise(MGG_ERR_INVALID_ARGUMENT, "bad sizes n=%d m=%d nn=%d", n, m, nn);
         if (!fused_chain_supported(m, nn))
             raise(MGG_ERR_UNSUPPORTED,
-                  "the allocation-free image chain runs the fused chains only (m = 128, 192, 256, 384, 512); "
-                  "m = %d needs rocFFT plans, which allocate", m);
+                  "the allocation-free image chain takes m = 128, 192, 256, 384 and 512 only, not m = %d", m);
         const size_t perImage = sizeof(float2) * (size_t)nn * (size_t)(m / 2 + 1);
         if (perImage > kNoAllocScratchBytes)
             raise(MGG_ERR_INVALID_ARGUMENT, "one image needs %zu scratch bytes, the fixed scratch holds %zu",

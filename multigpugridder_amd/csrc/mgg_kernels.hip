@@ -329,11 +329,10 @@ __device__ __forceinline__ int cvt_rpi(float x)
     return i;
 }
 
-// 501-entry table lookup (see bp_fast_kernel for the exactness argument),
-// read from the table in global memory (2 KB, cache-resident): the forward
-// kernel does only 15 lookups per pixel, and keeping the table out of LDS
-// leaves room for a fourth workgroup per CU.  Clamping the index to [0, 500]
-// picks the entry the reference's clamp of r would (|r| <= 2.5 here), and
+// 501-entry table lookup (see bp_fast_kernel for the exactness argument) from
+// the table in global memory (2 KB, cache-resident): 5-wide windows, and tiles
+// of 4-wide ones that cannot take the phase table.  Clamping the index to [0,
+// 500] picks the entry the reference's clamp of r would (|r| <= 2.5 here), and
 // keeps any index, even from a non-finite coordinate, inside the table.
 __device__ __forceinline__ float kb_fast_fp(const float *__restrict__ ker, float r)
 {
@@ -1202,7 +1201,7 @@ struct BPArgs {
     int maskD2;  // largest integer d2 with sqrtf((float)d2) <= maskR (-1: none)
     int posRound;  // bp_fast_kernel: in-mask voxels of orthonormal frames project to fi, fj >= 0.5
     int maskLo;    // smallest coordinate of an in-mask voxel (V/2 - floor(sqrt(maskD2)))
-    const int *order;  // bp_fast_kernel, bp_col_kernel: brick id per work item, heaviest first
+    const int *order;  // bp_fast_kernel, col_kernel: brick (block) id per work item, heaviest first
     unsigned perXcd, totalWork;
     const unsigned *check;  // bp_fast_kernel: launch_check_back's flag, or null
     float orthTol;          // frames that the column launches take are orthonormal to this
@@ -1368,7 +1367,7 @@ __global__ __launch_bounds__(kThreads) void bp_kernel(BPArgs p)
 // contributions go to a per-wave LDS accumulator one direction after the
 // other (plain read-modify-writes: a float LDS atomic holds the LDS for 194
 // cycles per wave, against 8; 7.58 -> 6.92 ms per 2,000 directions at N=128,
-// 2.67 -> 2.29 ms with the density, 777 at N=64); the four wave accumulators
+// 2.67 -> 2.29 ms with the density, 777 at N=64); the waves' accumulators
 // are combined in a fixed order at the end and added to the volume in FP64.
 //
 // Table index.  The reference, as contracted, takes
@@ -1544,7 +1543,7 @@ __global__ __launch_bounds__(64 * BFW) void bp_fast_kernel(BPArgs p)
         }
         __syncthreads();
 
-        // Directions of this chunk that wave wv handles: q = wv, wv+4, ...
+        // Directions of this chunk that wave wv handles: q = wv, wv + BFW, ...
         // Their active voxels stream through the wave's FIFO queue; every
         // full group of 64 entries is gathered with all lanes busy.
         int head = 0, tail = 0;  // queue indices (uniform), ring of size QCAP
@@ -1751,7 +1750,7 @@ __global__ __launch_bounds__(64 * BFW) void bp_fast_kernel(BPArgs p)
 // same distance from theirs), so lanes that meet one take each slot's index by
 // itself.
 //
-// Measured: 2,000 directions at N=128 6.9 (bp_fast_kernel) -> 6.35 ms, 1,000 at
+// Measured: 2,000 directions at N=128 6.9 (bp_fast_kernel) -> 6.3 ms, 1,000 at
 // N=96 3.0 -> 2.0 ms; the transpose of 2,048 at N=96 6.5 -> 5.6 ms.  Bound by
 // issue and LDS together: a pixel takes 37 vector instructions and five random
 // table reads (13.6 ns per wave and CU of the 14.6 measured), and another 40%
