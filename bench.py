@@ -51,7 +51,7 @@ def bytes_bp(m: int) -> int:
 
 
 def measured_traffic(path: str, n: int, kernel: str, chunk: int):
-    """HBM bytes per launch of the dominant kernel, from the committed rocprofv3
+    """Fabric bytes per launch of the dominant kernel, from the committed rocprofv3
     FETCH_SIZE + WRITE_SIZE summary (a line 'bytes_per_direction <kernel> N=<n>: <B>'),
     scaled to this run's directions per launch; None when not measured."""
     if not os.path.exists(path):
@@ -623,7 +623,7 @@ def main():
         # summed launch times; with several streams the chains overlap the projectors
         "kernel_ms_per_step": {k: round(kern[k][1], 3) for k in kern},
         "roofline": {
-            "kernel": "back_project (bp_kernel)" if dominant == "bp" else "forward_project (fp_kernel)",
+            "kernel": "back_project (col_kernel)" if dominant == "bp" else "forward_project (fp_lds_kernel)",
             "bound": "hbm",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
@@ -639,7 +639,7 @@ def main():
     # (125 per in-mask pixel and direction, the slab model's count for both
     # projectors: 5 x 5 x 5 per pixel forward, 25 per slab voxel back), FLOP at
     # 4 per tap (the weight product wi*wj*wk and the multiply-add into the sum)
-    # against the FP32 vector peak, and the HBM rate of the rocprof traffic per
+    # against the FP32 vector peak, and the rate of the rocprof fabric traffic per
     # direction at the live launch rate.
     taps = 125 * n_mask(m)
     rates = {"taps_per_direction": taps, "flops_per_tap": 4, "fp32_vector_peak_tflops": 157.3}
@@ -649,7 +649,7 @@ def main():
         tflops = 4 * taps * dps / 1e12
         rates[name] = {"directions_per_s": round(dps, 1), "taps_per_s": round(taps * dps, 1),
                        "tflops": round(tflops, 2), "frac_of_fp32_peak": round(tflops / 157.3, 4),
-                       "rocprof_hbm_gbs": round(tr * dps / 1e9, 1) if tr else None}
+                       "rocprof_fabric_gbs": round(tr * dps / 1e9, 1) if tr else None}
     out["rates"] = rates
     # Issue roofline: the projectors are gathers bound by instruction issue, so
     # their VALU rate (rocprof instruction count per direction x directions per

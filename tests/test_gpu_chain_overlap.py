@@ -23,7 +23,9 @@ def test_output_over_later_input(cuda):
 
     n, m, p = 16, 32, 600
     print(f"overlapping chain n={n} m={m} p={p}", flush=True)
-    cas = torch.randn((p, m, m), device=cuda)
+    g = torch.Generator(device=cuda)
+    g.manual_seed(6)
+    cas = torch.randn((p, m, m), device=cuda, generator=g)
     want = ops.cas_images_to_images(cas, n)
     out = torch.from_dlpack(cas[450:]).view(p, n, n)
     assert torch.equal(ops.cas_images_to_images(cas, n, out=out), want)
